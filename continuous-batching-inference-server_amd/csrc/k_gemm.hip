@@ -15,9 +15,9 @@
 // Two LDS buffers; the next K tile is fetched into registers while the
 // current one feeds the MFMAs (one barrier per K step).  Each wave owns a
 // (BM/WM) x (BN/WN) sub-tile of 32x32 MFMA blocks:
-//   bf16 / fp8:  v_mfma_f32_32x32x16_bf16 (fp8 weights are decoded to bf16
-//                exactly when stored to LDS; the per-channel scale is applied
-//                in the epilogue),
+//   bf16 / fp8:  v_mfma_f32_32x32x16_bf16 (fp8 weights are widened to bf16
+//                exactly, when stored to LDS or when a fragment is read from
+//                it; the per-channel scale is applied in the epilogue),
 //   fp32:        v_mfma_f32_32x32x2_f32, four per ds_read_b128 fragment.
 // Workgroups are renumbered so that each XCD (dispatch is round-robin over
 // the 8 XCDs) receives a contiguous run of tiles, M-tile fastest, so the
@@ -216,6 +216,21 @@ __device__ inline void epilogue_store_pre(const GemmArgs& g, int row, int col, f
   else ((float*)g.Y)[o] = v;
 }
 
+// 8 e4m3 codes (two dwords, lowest byte first) -> 8 bf16 with
+// v_cvt_scalef32_pk_bf16_fp8 (scale 1: exact, every e4m3 value is a bf16 value).
+__device__ inline bf16x8_t e4m3x8_to_bf16(uint32_t lo, uint32_t hi) {
+  const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+  const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+  const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+  const bf16x2_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+  uint4 u;
+  u.x = __builtin_bit_cast(uint32_t, a);
+  u.y = __builtin_bit_cast(uint32_t, b);
+  u.z = __builtin_bit_cast(uint32_t, c);
+  u.w = __builtin_bit_cast(uint32_t, d);
+  return __builtin_bit_cast(bf16x8_t, u);
+}
+
 template <typename WT>
 struct WLoad;  // global W chunk (covering 16 bytes of LDS) -> uint4 of the compute type
 template <>
@@ -237,14 +252,7 @@ struct WLoad<uint8_t> {
   typedef uint2 raw_t;
   static constexpr int EPC = 8;
   __device__ static inline raw_t load(const uint8_t* p) { return *(const uint2*)p; }
-  __device__ static inline uint4 cvt(const raw_t& r) {
-    uint4 o;
-    o.x = (uint32_t)e4m3_to_bf16(r.x & 0xFF) | ((uint32_t)e4m3_to_bf16((r.x >> 8) & 0xFF) << 16);
-    o.y = (uint32_t)e4m3_to_bf16((r.x >> 16) & 0xFF) | ((uint32_t)e4m3_to_bf16(r.x >> 24) << 16);
-    o.z = (uint32_t)e4m3_to_bf16(r.y & 0xFF) | ((uint32_t)e4m3_to_bf16((r.y >> 8) & 0xFF) << 16);
-    o.w = (uint32_t)e4m3_to_bf16((r.y >> 16) & 0xFF) | ((uint32_t)e4m3_to_bf16(r.y >> 24) << 16);
-    return o;
-  }
+  __device__ static inline uint4 cvt(const raw_t& r) { return __builtin_bit_cast(uint4, e4m3x8_to_bf16(r.x, r.y)); }
 };
 
 // Workgroup b is dispatched to XCD b % 8 (measured on gfx950 from the
@@ -618,7 +626,7 @@ __global__ __launch_bounds__(256) void splitk_layernorm_kernel(const GemmArgs g,
 }
 
 // ---------------------------------------------------------------------------
-// bf16 x bf16 on a multi-stage LDS ring fed by direct-to-LDS loads.
+// bf16 X times bf16 or fp8 W on a multi-stage LDS ring fed by direct-to-LDS loads.
 //
 // Each global_load_lds_dwordx4 moves 16 bytes per lane straight from global
 // memory into LDS at M0 + 16 * lane (no VGPRs, no ds_write): one wave
@@ -649,17 +657,123 @@ __device__ inline void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES>
+// One stage of the ring: BM rows of X (128 bytes of K = 64 bf16 each), then BN
+// rows of W (64 K elements: 128 bytes of bf16, or 64 bytes of e4m3 codes, which
+// stay codes in LDS and are widened when a fragment is read).  A 1 KiB DMA
+// instruction fills 8 rows of 128 bytes or 16 of 64; NP waves share a stage's
+// instructions, each the same number of X and of W ones.
+//
+// A 64-byte W row r keeps its 16-byte chunk c (codes 16 c .. + 15) in slot
+// c ^ ((r >> 2) & 3): the 16 lanes that a ds_read_b128 serves per cycle read one
+// chunk of 16 consecutive rows, i.e. four rows in each 64-byte quarter of the
+// 64 banks, in four distinct slots.  A lane's chunk covers two MFMA k steps
+// (codes 0..7 and 8..15), so with fp8 weights lane half h of k steps 2 j and
+// 2 j + 1 holds k = 32 j + 16 h + 0..7 and + 8..15, of W and X alike: every
+// product pairs the same k and only the order of the sum within 32 differs.
+//
+// The widening is 4 VALU instructions per 64 x 8 operand block, issued under
+// the MFMAs; keeping the codes in LDS halves the W bytes that the ring moves.
+// One mid-size layer (d 2048) at M = 512: 758 us on the register-staged
+// gemm_kernel with a scalar decode, 105 us here (qkv / out / fc1 / fc2 21 / 15 /
+// 23 / 29 us; 68 -> 493 TFLOP/s over the four calls, LayerNorms included).
+template <typename WT, int BM, int BN, int NP>
+struct DmaTile {
+  static constexpr bool FP8 = sizeof(WT) == 1;
+  static constexpr int WROW = 64 * (int)sizeof(WT);    // bytes of a W row per stage
+  static constexpr int WRPI = 1024 / WROW;             // W rows per instruction
+  static constexpr int LA = BM / 8 / NP, LB = BN / WRPI / NP, LPW = LA + LB;  // instructions per wave
+  static constexpr int A_BYTES = BM * 128, STAGE_BYTES = A_BYTES + BN * WROW;
+  static_assert(LA * 8 * NP == BM && LB * WRPI * NP == BN && BM % 16 == 0, "tile rows / waves");
+
+  // Wave p's lane sources (stage 0) and LDS byte offsets within a stage.
+  const uint8_t *a[LA], *b[LB];
+  __device__ DmaTile(const GemmArgs& g, int p, int lane, int m0, int n0, int kbeg) {
+#pragma unroll
+    for (int j = 0; j < LA; ++j) {
+      const int rr = (p * LA + j) * 8 + (lane >> 3);
+      a[j] = (const uint8_t*)((const uint16_t*)g.X + (int64_t)min(m0 + rr, g.M - 1) * g.ldx + kbeg +
+                              swz_slot(rr, lane & 7) * 8);
+    }
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+      const int rr = (p * LB + j) * WRPI + lane / (WROW / 16);
+      const int chunk = FP8 ? (lane & 3) ^ ((rr >> 2) & 3) : swz_slot(rr, lane & 7);
+      b[j] = (const uint8_t*)((const WT*)g.W + (int64_t)min(n0 + rr, g.N - 1) * g.ldw + kbeg) + chunk * 16;
+    }
+  }
+  __device__ static int a_ofs(int p, int j) { return (p * LA + j) * 1024; }
+  __device__ static int b_ofs(int p, int j) { return A_BYTES + (p * LB + j) * 1024; }
+  // Issues this wave's loads of K tile kt into the stage at LDS address base.
+  __device__ void issue(int p, int kt, uint32_t base) const {
+#pragma unroll
+    for (int j = 0; j < LA; ++j) lds_dma16(a[j] + kt * 128, base + a_ofs(p, j));
+#pragma unroll
+    for (int j = 0; j < LB; ++j) lds_dma16(b[j] + kt * WROW, base + b_ofs(p, j));
+  }
+};
+
+// Waits until a wave's loads of a K tile have landed, with `younger` (< STAGES)
+// tiles of LPW loads each issued after it.
+template <int LPW, int STAGES>
+__device__ inline void wait_dma_tile(int younger) {
+  static_assert(STAGES >= 2 && STAGES <= 8 && LPW * (STAGES - 1) < 64, "vmcnt range");
+  if constexpr (STAGES > 7) { if (younger >= 7) { wait_vmcnt<7 * LPW>(); return; } }
+  if constexpr (STAGES > 6) { if (younger >= 6) { wait_vmcnt<6 * LPW>(); return; } }
+  if constexpr (STAGES > 5) { if (younger >= 5) { wait_vmcnt<5 * LPW>(); return; } }
+  if constexpr (STAGES > 4) { if (younger >= 4) { wait_vmcnt<4 * LPW>(); return; } }
+  if constexpr (STAGES > 3) { if (younger >= 3) { wait_vmcnt<3 * LPW>(); return; } }
+  if constexpr (STAGES > 2) { if (younger >= 2) { wait_vmcnt<2 * LPW>(); return; } }
+  if (younger >= 1) wait_vmcnt<LPW>();
+  else wait_vmcnt<0>();
+}
+
+// The MFMA operands of one wave's (32 FM) x (32 FN) sub-tile for the 16-wide k
+// steps of a stage, double-buffered: load(ks + 1) may be issued before the
+// MFMAs of step ks.
+template <typename T, int FM, int FN>
+struct DmaFrags {
+  static constexpr bool FP8 = T::FP8;
+  bf16x8_t a[2][FM];
+  uint4 b[2][FN];  // bf16: per k step; fp8: 16 codes, per pair of k steps
+  int a_row, b_row, half, sw, sw4;  // sw, sw4: swizzle keys of every row this lane reads (l32 plus multiples of 32)
+  __device__ DmaFrags(int m_row, int n_row, int lane)
+      : a_row((m_row + (lane & 31)) * 128), b_row(T::A_BYTES + (n_row + (lane & 31)) * T::WROW), half(lane >> 5),
+        sw(((lane & 31) >> 1) & 7), sw4(((lane & 31) >> 2) & 3) {}
+  __device__ void load(const uint8_t* stage, int ks) {
+    const int ka = FP8 ? 4 * (ks >> 1) + 2 * half + (ks & 1) : 2 * ks + half;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) a[ks & 1][i] = *(const bf16x8_t*)(stage + a_row + i * 32 * 128 + ((ka ^ sw) << 4));
+    if (FP8 && (ks & 1)) return;
+    const int kb = FP8 ? ((ks + half) ^ sw4) << 4 : (ka ^ sw) << 4;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) b[FP8 ? ks >> 1 : ks & 1][j] = *(const uint4*)(stage + b_row + j * 32 * T::WROW + kb);
+  }
+  __device__ void mfma(int ks, f32x16_t (&acc)[FM][FN]) const {
+    bf16x8_t w[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      if constexpr (FP8) {
+        const uint4 r = b[ks >> 1][j];
+        w[j] = (ks & 1) ? e4m3x8_to_bf16(r.z, r.w) : e4m3x8_to_bf16(r.x, r.y);
+      } else {
+        w[j] = __builtin_bit_cast(bf16x8_t, b[ks & 1][j]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks & 1][i], w[j], acc[i][j], 0, 0, 0);
+  }
+};
+
+template <typename WT, int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
   constexpr int NWAVES = WM * WN;
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int FM = TM / 32, FN = TN / 32;
-  constexpr int ROWS = BM + BN;                 // tile rows per stage (A then B)
-  constexpr int GROUPS = ROWS / 8;              // 1 KiB DMA instructions per stage
-  constexpr int LPW = GROUPS / NWAVES;          // per wave
-  constexpr int STAGE_BYTES = ROWS * 128;
-  static_assert(LPW * NWAVES == GROUPS && BM % 8 == 0 && BN % 8 == 0, "tile / wave mismatch");
-  static_assert(LPW * (STAGES - 1) < 64, "vmcnt range");
+  typedef DmaTile<WT, BM, BN, NWAVES> T;
+  constexpr int LPW = T::LPW, STAGE_BYTES = T::STAGE_BYTES;
 
   constexpr int RING = STAGES * STAGE_BYTES;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[RING > parked_bytes<BM, BN>() ? RING : parked_bytes<BM, BN>()];
@@ -672,33 +786,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wn = wave / WM;
-  const int half = lane >> 5, l32 = lane & 31;
 
-  // Per-lane source pointers of this wave's DMA instructions (k tile 0).
-  const uint16_t* src[LPW];
-#pragma unroll
-  for (int j = 0; j < LPW; ++j) {
-    const int grp = wave * LPW + j;
-    const int rr = grp * 8 + (lane >> 3);
-    const int chunk = swz_slot(rr, lane & 7);  // the chunk that belongs in slot lane & 7 of row rr
-    if (rr < BM) {
-      const int r = min(m0 + rr, g.M - 1);
-      src[j] = (const uint16_t*)g.X + (int64_t)r * g.ldx + kbeg + chunk * 8;
-    } else {
-      const int r = min(n0 + rr - BM, g.N - 1);
-      src[j] = (const uint16_t*)g.W + (int64_t)r * g.ldw + kbeg + chunk * 8;
-    }
-  }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * LPW * 1024);
-
-  auto issue = [&](int kt) {
-    const uint32_t base = wave_lds + (uint32_t)((kt % STAGES) * STAGE_BYTES);
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) lds_dma16(src[j] + kt * 64, base + j * 1024);
-  };
+  const T src(g, wave, lane, m0, n0, kbeg);
+  const uint32_t lds0 =
+      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem);
+  auto issue = [&](int kt) { src.issue(wave, kt, lds0 + (uint32_t)((kt % STAGES) * STAGE_BYTES)); };
 
   f32x16_t acc[FM][FN];
 #pragma unroll
@@ -708,37 +802,14 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  // Fragment byte offsets inside a stage: swz(row, kc); every fragment row
-  // this lane reads is l32 plus a multiple of 32, so its swizzle key is l32's.
-  const int a_row0 = (wm * TM + l32) * 128;
-  const int b_row0 = (BM + wn * TN + l32) * 128;
-  const int sw = (l32 >> 1) & 7;
-  bf16x8_t af[2][FM], bf[2][FN];
-  auto load_frags = [&](int slot, int ks, int fb) {
-    const uint8_t* st = smem + slot * STAGE_BYTES;
-    const int kc = ((2 * ks + half) ^ sw) << 4;
-#pragma unroll
-    for (int i = 0; i < FM; ++i) af[fb][i] = *(const bf16x8_t*)(st + a_row0 + i * 32 * 128 + kc);
-#pragma unroll
-    for (int j = 0; j < FN; ++j) bf[fb][j] = *(const bf16x8_t*)(st + b_row0 + j * 32 * 128 + kc);
-  };
+  DmaFrags<T, FM, FN> fr(wm * TM, wn * TN, lane);
   // Waits until k tile t has landed in LDS for every wave: at most
   // (last - t) * LPW of this wave's DMA loads may remain (tiles t+1..last are
   // the younger ones in flight), then a barrier.  The lgkmcnt wait makes
   // every wave's earlier ds_reads complete before any wave refills the slot
   // they read.
   auto await_tile = [&](int t, int last) {
-    const int younger = last - t;
-    if constexpr (STAGES >= 4) {
-      if (younger >= 3) wait_vmcnt<3 * LPW>();
-      else if (younger == 2) wait_vmcnt<2 * LPW>();
-      else if (younger == 1) wait_vmcnt<LPW>();
-      else wait_vmcnt<0>();
-    } else {
-      if (younger >= 2) wait_vmcnt<2 * LPW>();
-      else if (younger == 1) wait_vmcnt<LPW>();
-      else wait_vmcnt<0>();
-    }
+    wait_dma_tile<LPW, STAGES>(last - t);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
   };
@@ -748,45 +819,41 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
   for (int t = 0; t < STAGES; ++t)
     if (t < KT) issue(t);
   await_tile(0, min(KT - 1, STAGES - 1));
-  load_frags(0, 0, 0);
+  fr.load(smem, 0);
 
   // The fragments of sub-step ks+1 are read while sub-step ks's MFMAs run;
   // across a tile boundary the barrier sits between the last sub-step's
   // fragment reads and its MFMAs, and the freed slot is refilled with tile
   // kt + STAGES right after it.
   for (int kt = 0; kt < KT; ++kt) {
-    const int slot = kt % STAGES;
+    const uint8_t* stage = smem + (kt % STAGES) * STAGE_BYTES;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      const int fb = ks & 1;
       if (ks < 3) {
-        load_frags(slot, ks + 1, fb ^ 1);
+        fr.load(stage, ks + 1);
       } else if (kt + 1 < KT) {
         await_tile(kt + 1, min(KT - 1, kt + STAGES - 1));
         if (kt + STAGES < KT) issue(kt + STAGES);
-        load_frags((kt + 1) % STAGES, 0, fb ^ 1);
+        fr.load(smem + ((kt + 1) % STAGES) * STAGE_BYTES, 0);
       }
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[fb][i], bf[fb][j], acc[i][j], 0, 0, 0);
+      fr.mfma(ks, acc);
     }
   }
 
   epilogue_parked<BM, BN, WM, WN>(g, kz, smem, acc, m0, n0);
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES>
+template <typename WT, int BM, int BN, int WM, int WN, int STAGES>
 int launch_dma(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = cdiv(g.M, BM) * cdiv(g.N, BN);
-  gemm_bf16_dma_kernel<BM, BN, WM, WN, STAGES><<<dim3((unsigned)tiles, 1, g.ksplit), WM * WN * 64, 0, s>>>(with_vec(g));
+  gemm_bf16_dma_kernel<WT, BM, BN, WM, WN, STAGES>
+      <<<dim3((unsigned)tiles, 1, g.ksplit), WM * WN * 64, 0, s>>>(with_vec(g));
   return check_launch("cbis_gemm(bf16)");
 }
 
 // ---------------------------------------------------------------------------
-// bf16 x bf16, wave-specialised, for grids of at least half a CU count of
-// 128 x 128 tiles.
+// bf16 X times bf16 or fp8 W, wave-specialised, for grids of at least half a
+// CU count of 128 x 128 tiles.
 //
 // 8 waves, one workgroup per CU.  Waves 0-3 (one per SIMD) are consumers:
 // they only read fragments from LDS and issue MFMAs, each on a
@@ -815,15 +882,13 @@ int launch_dma(const GemmArgs& g, hipStream_t s) {
 // ---------------------------------------------------------------------------
 constexpr int kWsProducers = 4;
 
-template <int BM, int BN, int STAGES, int WM>
+template <typename WT, int BM, int BN, int STAGES, int WM>
 struct WsTile {
+  typedef DmaTile<WT, BM, BN, kWsProducers> Dma;
   static constexpr int WN = 4 / WM;                    // consumers as WM x WN
   static constexpr int TM = BM / WM, TN = BN / WN;
   static constexpr int FM = TM / 32, FN = TN / 32;
-  static constexpr int ROWS = BM + BN;
-  static constexpr int LPW = ROWS / 8 / kWsProducers;  // 1 KiB DMA instructions per producer per tile
-  static constexpr int STAGE_BYTES = ROWS * 128;
-  static constexpr int RING = STAGES * STAGE_BYTES;
+  static constexpr int RING = STAGES * Dma::STAGE_BYTES;
   static constexpr int PITCH = BN + 8;                 // floats per parked output row
   static constexpr int kLdsMax = 160 * 1024;
   // The accumulators are parked PH row blocks at a time when the whole tile
@@ -833,8 +898,6 @@ struct WsTile {
   static constexpr int PARK = PR * PITCH * 4;
   static constexpr int LDS = RING > PARK ? RING : PARK;
   static_assert(WM * WN == 4 && TM % 32 == 0 && TN % 32 == 0, "consumer layout");
-  static_assert(LPW * 8 * kWsProducers == ROWS, "tile rows / producers");
-  static_assert(LPW * (STAGES - 1) < 64, "vmcnt range");
   static_assert(BM % PH == 0 && PR * PITCH * 4 <= kLdsMax && LDS <= kLdsMax, "LDS");
 };
 
@@ -1125,10 +1188,11 @@ __device__ inline void epilogue_top2(const GemmArgs& g, const Top2Cols<BN>& cc, 
   else epilogue_top2_rows<BM, BN, NT, false, false>(g, cc, tile, pitch, m0, n0, tid);
 }
 
-template <int BM, int BN, int STAGES, int REGS, int WM, bool TOP2>
+template <typename WT, int BM, int BN, int STAGES, int REGS, int WM, bool TOP2>
 __global__ __launch_bounds__(512) void gemm_bf16_ws_kernel(const GemmArgs g) {
-  typedef WsTile<BM, BN, STAGES, WM> T;
-  constexpr int LPW = T::LPW, STAGE_BYTES = T::STAGE_BYTES, FM = T::FM, FN = T::FN;
+  typedef WsTile<WT, BM, BN, STAGES, WM> T;
+  typedef typename T::Dma Dma;
+  constexpr int LPW = Dma::LPW, STAGE_BYTES = Dma::STAGE_BYTES, FM = T::FM, FN = T::FN;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[T::LDS];
 
   const int2 tt = tile_of<BM, BN>(g, xcd_contiguous(blockIdx.x, gridDim.x));
@@ -1144,42 +1208,20 @@ __global__ __launch_bounds__(512) void gemm_bf16_ws_kernel(const GemmArgs g) {
   f32x16_t acc[FM][FN];
 
   if (wave >= 4) {
-    // Producer: tile rows p*8*LPW .. of every stage (A rows first, then B).
+    // Producer.
     const int p = wave - 4;
-    const uint16_t* src[LPW];
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) {
-      const int rr = (p * LPW + j) * 8 + (lane >> 3);
-      const int chunk = swz_slot(rr, lane & 7);  // the chunk that belongs in slot lane & 7 of row rr
-      if (rr < BM) src[j] = (const uint16_t*)g.X + (int64_t)min(m0 + rr, g.M - 1) * g.ldx + kbeg + chunk * 8;
-      else src[j] = (const uint16_t*)g.W + (int64_t)min(n0 + rr - BM, g.N - 1) * g.ldw + kbeg + chunk * 8;
-    }
+    const Dma src(g, p, lane, m0, n0, kbeg);
     if constexpr (REGS == 0) {
-      const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-      const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds0 + p * LPW * 1024);
-      auto issue = [&](int kt) {
-        const uint32_t base = wave_lds + (uint32_t)((kt % STAGES) * STAGE_BYTES);
-#pragma unroll
-        for (int j = 0; j < LPW; ++j) lds_dma16(src[j] + kt * 64, base + j * 1024);
-      };
-      // Waits for a tile with `younger` tiles issued after it.
-      auto wait_tile = [&](int younger) {
-        if constexpr (STAGES >= 4) {
-          if (younger >= 3) { wait_vmcnt<3 * LPW>(); return; }
-        }
-        if constexpr (STAGES >= 3) {
-          if (younger >= 2) { wait_vmcnt<2 * LPW>(); return; }
-        }
-        if (younger >= 1) wait_vmcnt<LPW>();
-        else wait_vmcnt<0>();
-      };
+      const uint32_t lds0 =
+          __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem);
+      auto issue = [&](int kt) { src.issue(p, kt, lds0 + (uint32_t)((kt % STAGES) * STAGE_BYTES)); };
 #pragma unroll
       for (int t = 0; t < STAGES; ++t)
         if (t < KT) issue(t);
-      wait_tile(min(KT - 1, STAGES - 1));
+      wait_dma_tile<LPW, STAGES>(min(KT - 1, STAGES - 1));
       asm volatile("s_barrier" ::: "memory");
       for (int kt = 0; kt + 1 < KT; ++kt) {
-        wait_tile(min(KT - 1, kt + STAGES - 1) - (kt + 1));
+        wait_dma_tile<LPW, STAGES>(min(KT - 1, kt + STAGES - 1) - (kt + 1));
         asm volatile("s_barrier" ::: "memory");
         if (kt + STAGES < KT) issue(kt + STAGES);
       }
@@ -1192,14 +1234,19 @@ __global__ __launch_bounds__(512) void gemm_bf16_ws_kernel(const GemmArgs g) {
       // j + STAGES - 1 + REGS; its ds_writes finish before barrier j + 1.
       static_assert(STAGES >= 2 && STAGES - 1 <= REGS, "register ring shorter than the LDS lead");
       u32x4_t regs[REGS][LPW];
-      uint8_t* my_lds = smem + p * LPW * 1024 + lane * 16;
+      uint8_t* my_lds = smem + lane * 16;
       auto load = [&](int r, int t) {
 #pragma unroll
-        for (int j = 0; j < LPW; ++j) regs[r][j] = *(const u32x4_t*)(src[j] + t * 64);
+        for (int j = 0; j < Dma::LA; ++j) regs[r][j] = *(const u32x4_t*)(src.a[j] + t * 128);
+#pragma unroll
+        for (int j = 0; j < Dma::LB; ++j) regs[r][Dma::LA + j] = *(const u32x4_t*)(src.b[j] + t * Dma::WROW);
       };
       auto store = [&](int r, int t) {
+        uint8_t* st = my_lds + (t % STAGES) * STAGE_BYTES;
 #pragma unroll
-        for (int j = 0; j < LPW; ++j) *(u32x4_t*)(my_lds + (t % STAGES) * STAGE_BYTES + j * 1024) = regs[r][j];
+        for (int j = 0; j < Dma::LA; ++j) *(u32x4_t*)(st + Dma::a_ofs(p, j)) = regs[r][j];
+#pragma unroll
+        for (int j = 0; j < Dma::LB; ++j) *(u32x4_t*)(st + Dma::b_ofs(p, j)) = regs[r][Dma::LA + j];
       };
 #pragma unroll
       for (int r = 0; r < REGS; ++r)
@@ -1237,48 +1284,35 @@ __global__ __launch_bounds__(512) void gemm_bf16_ws_kernel(const GemmArgs g) {
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    const int a_row0 = (wm * T::TM + l32) * 128;
-    const int b_row0 = (BM + wn * T::TN + l32) * 128;
-    const int sw = (l32 >> 1) & 7;  // swizzle key of every fragment row this lane reads
-    bf16x8_t af[2][FM], bf[2][FN];
-    auto load_frags = [&](int slot, int ks, int fb) {
-      const uint8_t* st = smem + slot * STAGE_BYTES;
-      const int kc = ((2 * ks + half) ^ sw) << 4;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) af[fb][i] = *(const bf16x8_t*)(st + a_row0 + i * 32 * 128 + kc);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) bf[fb][j] = *(const bf16x8_t*)(st + b_row0 + j * 32 * 128 + kc);
-    };
+    DmaFrags<Dma, FM, FN> fr(wm * T::TM, wn * T::TN, lane);
     asm volatile("s_barrier" ::: "memory");
-    load_frags(0, 0, 0);
+    fr.load(smem, 0);
     for (int kt = 0; kt < KT; ++kt) {
-      const int slot = kt % STAGES;
+      const uint8_t* stage = smem + (kt % STAGES) * STAGE_BYTES;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const int fb = ks & 1;
         if (ks < 3) {
-          load_frags(slot, ks + 1, fb ^ 1);
+          fr.load(stage, ks + 1);
         } else if (kt + 1 < KT) {
           asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-          load_frags((kt + 1) % STAGES, 0, fb ^ 1);
+          fr.load(smem + ((kt + 1) % STAGES) * STAGE_BYTES, 0);
         }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[fb][i], bf[fb][j], acc[i][j], 0, 0, 0);
+        fr.mfma(ks, acc);
         // Issue the next sub-step's fragment reads between this sub-step's
         // MFMAs, one read after each MFMA, so they land while the MFMAs run
         // (left to itself the scheduler sinks them below the MFMAs and the
         // next sub-step waits on them: qkv 41.3 -> 40.1 us, fc1 50.4 -> 48.5).
-        constexpr int kReads = FM + FN, kMfma = FM * FN, kPairs = kReads < kMfma ? kReads : kMfma;
+        constexpr int kMfma = FM * FN;
+        const int reads = FM + ((Dma::FP8 && (ks & 1) == 0) ? 0 : FN), pairs = reads < kMfma ? reads : kMfma;
 #pragma unroll
-        for (int q = 0; q < kPairs; ++q) {
+        for (int q = 0; q < pairs; ++q) {
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
         }
-        if constexpr (kMfma > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kPairs, 0);
-        if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
+#pragma unroll
+        for (int q = pairs; q < kMfma; ++q) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+        for (int q = pairs; q < reads; ++q) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
     }
     __builtin_amdgcn_s_setprio(0);
@@ -1311,11 +1345,14 @@ __global__ __launch_bounds__(512) void gemm_bf16_ws_kernel(const GemmArgs g) {
   }
 }
 
-template <int BM, int BN, int STAGES, int REGS = 0, int WM = 2>
+template <typename WT, int BM, int BN, int STAGES, int REGS = 0, int WM = 2>
 int launch_ws(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = cdiv(g.M, BM) * cdiv(g.N, BN);
-  if (g.amax) gemm_bf16_ws_kernel<BM, BN, STAGES, REGS, WM, true><<<dim3((unsigned)tiles, 1, 1), 512, 0, s>>>(g);
-  else gemm_bf16_ws_kernel<BM, BN, STAGES, REGS, WM, false><<<dim3((unsigned)tiles, 1, g.ksplit), 512, 0, s>>>(with_vec(g));
+  if (g.amax)
+    gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, true><<<dim3((unsigned)tiles, 1, 1), 512, 0, s>>>(g);
+  else
+    gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, false>
+        <<<dim3((unsigned)tiles, 1, g.ksplit), 512, 0, s>>>(with_vec(g));
   return check_launch("cbis_gemm(bf16 ws)");
 }
 
@@ -1336,33 +1373,6 @@ int launch_ws(const GemmArgs& g, hipStream_t s) {
 //            16-k block in element e of a float4, one MFMA per e.
 // C fragment: lane l holds rows 4 * (l / 16) + i, column l % 16.
 // ---------------------------------------------------------------------------
-template <typename WT>
-struct SkinnyW;
-template <>
-struct SkinnyW<uint16_t> {  // bf16: 8 elements = 16 bytes
-  __device__ static inline bf16x8_t load(const uint16_t* p) { return *(const bf16x8_t*)p; }
-};
-template <>
-struct SkinnyW<uint8_t> {  // fp8 e4m3: 8 elements = 8 bytes
-  __device__ static inline bf16x8_t load(const uint8_t* p) {
-    const uint2 r = *(const uint2*)p;
-    return load_pair(r.x, r.y);
-  }
-  // 8 e4m3 codes (two dwords, lowest byte first) -> 8 bf16.
-  __device__ static inline bf16x8_t load_pair(uint32_t lo, uint32_t hi) {
-    const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
-    const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
-    const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
-    const bf16x2_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
-    uint4 u;
-    u.x = __builtin_bit_cast(uint32_t, a);
-    u.y = __builtin_bit_cast(uint32_t, b);
-    u.z = __builtin_bit_cast(uint32_t, c);
-    u.w = __builtin_bit_cast(uint32_t, d);
-    return __builtin_bit_cast(bf16x8_t, u);
-  }
-};
-
 constexpr int kSkinnyWaves = 8;
 
 template <typename XT, typename WT, int MB, bool LN>
@@ -1549,8 +1559,8 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny_kernel(const Ge
       }
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
-        const bf16x8_t w0 = SkinnyW<uint8_t>::load_pair(wr[u].x, wr[u].y);
-        const bf16x8_t w1 = SkinnyW<uint8_t>::load_pair(wr[u].z, wr[u].w);
+        const bf16x8_t w0 = e4m3x8_to_bf16(wr[u].x, wr[u].y);
+        const bf16x8_t w1 = e4m3x8_to_bf16(wr[u].z, wr[u].w);
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
           acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u][i][0], w0, acc[i], 0, 0, 0);
@@ -1571,7 +1581,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny_kernel(const Ge
       bf16x8_t w[NU], x[NU][MB];
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
-        w[u] = SkinnyW<WT>::load(wp + (kb + u) * KB);
+        w[u] = *(const bf16x8_t*)(wp + (kb + u) * KB);
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
           if constexpr (LN) x[u][i] = ln_bf16x8(i, (kb + u) * KB + 8 * q);
@@ -1734,7 +1744,7 @@ struct SplitPlan {
   int k_per = 0;
 };
 
-// Kernel for a bf16 x bf16 problem on the direct-to-LDS paths, from the
+// Kernel for a bf16 or fp8 W on the direct-to-LDS paths, from the
 // tile counts (measured on config 4's shapes at M = 1216, TFLOP/s):
 //   < kCUs / 2 tiles of 128 x 128, or K < 512: gemm_bf16_dma_kernel, 64 x 64
 //     tiles or 128 x 128 with split-K (plan_dma_split); with under 8 K tiles
@@ -1827,8 +1837,8 @@ SplitPlan plan_skinny_split(int M, int N, int K, int w_dtype) {
 }
 
 bool dma_eligible(const cbis_gemm_desc* d) {
-  return d->x_dtype == CBIS_BF16 && d->w_dtype == CBIS_BF16 && ((uintptr_t)d->W & 15u) == 0 &&
-         (d->ldw * 2) % 16 == 0;
+  return d->x_dtype == CBIS_BF16 && ((uintptr_t)d->W & 15u) == 0 &&
+         (d->w_dtype == CBIS_BF16 ? d->ldw * 2 : d->ldw) % 16 == 0;
 }
 
 template <int BM, int BN, int WM, int WN, typename XT, typename WT>
@@ -1893,16 +1903,44 @@ int dispatch(const GemmArgs& g, hipStream_t s) {
   }
 }
 
+// Launches the direct-to-LDS kernel that choose_bf16 picks, on g's split.
+template <typename WT>
+int dispatch_dma(const GemmArgs& g, hipStream_t s) {
+  const bool split = g.ksplit > 1;
+  switch (choose_bf16(g.M, g.N, g.K)) {
+    case Bf16Path::kWs256: return launch_ws<WT, 128, 256, 3>(g, s);
+    case Bf16Path::kWs160: return launch_ws<WT, 160, 256, 3, 0, 1>(g, s);
+    case Bf16Path::kWs128: return launch_ws<WT, 128, 128, 3>(g, s);
+    case Bf16Path::kWs96: return launch_ws<WT, 96, 128, 3, 0, 1>(g, s);
+    case Bf16Path::kWs160Split:
+      return split ? launch_ws<WT, 160, 256, 3, 0, 1>(g, s) : launch_ws<WT, 96, 128, 3, 0, 1>(g, s);
+    case Bf16Path::kWs128R:
+      if constexpr (sizeof(WT) == 2) return launch_ws<WT, 128, 128, 2, 3>(g, s);
+      else return launch_ws<WT, 128, 128, 3>(g, s);
+    case Bf16Path::kSmall: break;
+  }
+  // Grids with fewer 128 x 128 tiles than CUs run 64 x 64 tiles (4 waves
+  // of 32 x 32): four times the workgroups (config 4's out-projection,
+  // 160 tiles: 28.3 -> 23.4 us).  A third ring slot pays when the grid
+  // fills the CUs and K has 8 or more tiles (config 2's MLP down at
+  // M = 4096, K = 1024: 12.2 -> 10.7 us; at M = 512 it costs 1 us).
+  if (!split && cdiv(g.M, kDmaBM) * cdiv(g.N, kDmaBN) < kCUs) {
+    if (g.K >= 512 && cdiv(g.M, 64) * cdiv(g.N, 64) >= kCUs) return launch_dma<WT, 64, 64, 2, 2, 3>(g, s);
+    return launch_dma<WT, 64, 64, 2, 2, 2>(g, s);
+  }
+  return launch_dma<WT, kDmaBM, kDmaBN, 2, 4, 2>(g, s);
+}
+
 // Column-tile width of the greedy-mode partials for d's GEMM path: the
 // kernels that reduce in their epilogue are the skinny one (16 columns per
-// workgroup) and the wave-specialised bf16 ones (their BN); 0 for the others
-// (fp32 or fp8 weights at M > 64, small bf16 grids), whose logits
+// workgroup) and the wave-specialised ones (their BN); 0 for the others
+// (fp32 weights at M > 64, small grids, unaligned W), whose logits
 // cbis_gemm_argmax stores and reduces instead.  Follows gemm_run's choice.
 int argmax_tile_cols(const cbis_gemm_desc* d) {
   const int we = d->w_dtype == CBIS_F32 ? 4 : (d->w_dtype == CBIS_BF16 ? 2 : 1);
   const bool w_al = ((uintptr_t)d->W & 15u) == 0 && (d->ldw * we) % 16 == 0;
   if (d->M <= kSkinnyMaxM && w_al && d->K % (d->w_dtype == CBIS_FP8E4M3 ? 64 : 32) == 0) return 16;
-  if (d->x_dtype != CBIS_BF16 || d->w_dtype != CBIS_BF16 || !dma_eligible(d)) return 0;
+  if (!dma_eligible(d)) return 0;
   switch (choose_bf16(d->M, d->N, d->K)) {
     case Bf16Path::kWs256:
     case Bf16Path::kWs160: return 256;
@@ -1945,7 +1983,7 @@ bool skinny_path(const cbis_gemm_desc* d) {
 // us skinny, 4.2 / 4.2 / 4.7 / 7.0 tiled).  fp32 weights keep the skinny
 // kernel (M = 64 qkv 8.3 us against 9.1 on the fp32 tiles), fp8 weights too.
 bool plain_skinny(const cbis_gemm_desc* d) {
-  return skinny_path(d) && (d->M <= 32 || !dma_eligible(d));
+  return skinny_path(d) && (d->M <= 32 || d->w_dtype != CBIS_BF16 || !dma_eligible(d));
 }
 
 // Whether cbis_layernorm_gemm(_argmax) forms d's LayerNorm inside the GEMM.
@@ -2042,42 +2080,18 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
     }
     return dispatch<float, float>(g, s);
   }
-  if (d->w_dtype == CBIS_BF16) {
-    // The direct-to-LDS path needs 16-byte aligned rows of both operands.
-    if (dma_eligible(d)) {
-      const Bf16Path path = choose_bf16(d->M, d->N, d->K);
-      const SplitPlan p = plan_dma_split(d->M, d->N, d->K);
-      const size_t need = (size_t)p.ksplit * d->M * d->N * sizeof(float);
-      const bool split = !amax && p.ksplit > 1 && d->workspace && d->workspace_bytes >= need;
-      if (split) {
-        g.ksplit = p.ksplit;
-        g.k_per = p.k_per;
-        g.partial = (float*)d->workspace;
-      }
-      switch (path) {
-        case Bf16Path::kWs256: return launch_ws<128, 256, 3>(g, s);
-        case Bf16Path::kWs160: return launch_ws<160, 256, 3, 0, 1>(g, s);
-        case Bf16Path::kWs128: return launch_ws<128, 128, 3>(g, s);
-        case Bf16Path::kWs96: return launch_ws<96, 128, 3, 0, 1>(g, s);
-        case Bf16Path::kWs160Split:
-          return split ? launch_ws<160, 256, 3, 0, 1>(g, s) : launch_ws<96, 128, 3, 0, 1>(g, s);
-        case Bf16Path::kWs128R: return launch_ws<128, 128, 2, 3>(g, s);
-        case Bf16Path::kSmall: break;
-      }
-      // Grids with fewer 128 x 128 tiles than CUs run 64 x 64 tiles (4 waves
-      // of 32 x 32): four times the workgroups (config 4's out-projection,
-      // 160 tiles: 28.3 -> 23.4 us).  A third ring slot pays when the grid
-      // fills the CUs and K has 8 or more tiles (config 2's MLP down at
-      // M = 4096, K = 1024: 12.2 -> 10.7 us; at M = 512 it costs 1 us).
-      if (g.ksplit == 1 && cdiv(d->M, kDmaBM) * cdiv(d->N, kDmaBN) < kCUs) {
-        if (d->K >= 512 && cdiv(d->M, 64) * cdiv(d->N, 64) >= kCUs) return launch_dma<64, 64, 2, 2, 3>(g, s);
-        return launch_dma<64, 64, 2, 2, 2>(g, s);
-      }
-      return launch_dma<kDmaBM, kDmaBN, 2, 4, 2>(g, s);
+  // The direct-to-LDS path needs 16-byte aligned rows of both operands.
+  if (dma_eligible(d)) {
+    const SplitPlan p = plan_dma_split(d->M, d->N, d->K);
+    const size_t need = (size_t)p.ksplit * d->M * d->N * sizeof(float);
+    if (!amax && p.ksplit > 1 && d->workspace && d->workspace_bytes >= need) {
+      g.ksplit = p.ksplit;
+      g.k_per = p.k_per;
+      g.partial = (float*)d->workspace;
     }
-    return dispatch<uint16_t, uint16_t>(g, s);
+    return d->w_dtype == CBIS_BF16 ? dispatch_dma<uint16_t>(g, s) : dispatch_dma<uint8_t>(g, s);
   }
-  return dispatch<uint16_t, uint8_t>(g, s);
+  return d->w_dtype == CBIS_BF16 ? dispatch<uint16_t, uint16_t>(g, s) : dispatch<uint16_t, uint8_t>(g, s);
 }
 
 int gemm_argmax(const cbis_gemm_desc* d, int* next_token, float* margin, void* workspace, size_t workspace_bytes,

@@ -515,6 +515,52 @@ def test_gemm_fp8_weights(cbis, oracle, dev, M):
     assert np.abs(Y.cpu().numpy() - ref).max() < FP32_TOL
 
 
+@pytest.mark.parametrize("M,N,K,gelu,res", [
+    (65, 250, 64, True, False),       # 64 x 64 tiles, one K tile, ragged rows and columns
+    (700, 1000, 576, False, True),    # 64 x 64 tiles, three ring slots
+    (200, 1000, 4096, True, False),   # 128 x 128 tiles, split K
+    (1216, 2050, 512, False, True),   # wave-specialised 96 x 128, ragged last column group
+    (300, 8200, 512, True, False),    # wave-specialised 128 x 128
+    (1300, 8192, 512, False, False),  # the same, over two tiles per CU
+    (1216, 6144, 512, False, True),   # wave-specialised 128 x 256
+    (1217, 8192, 576, True, False),   # wave-specialised 160 x 256, parked in two row blocks
+    (1216, 2048, 6144, False, True),  # wave-specialised 160 x 256, split K
+])
+def test_gemm_fp8_tiles(cbis, oracle, dev, M, N, K, gelu, res):
+    """fp8 weights at M > 64 on every direct-to-LDS tile (e4m3 codes in the
+    ring, widened at the fragment read), against the product in 64 bits on
+    sampled rows.  Codes and bf16 X are exact, each of the K + 3 fp32
+    operations of an output (sum, scale, bias, residual) is at most 2^-23 of
+    the sum of magnitudes off, GELU (slope <= 1.13) adds 1e-6 relative."""
+    import torch
+    codes, sc = oracle.quantize_e4m3_rows(oracle.normal(81, 2, N * K, 0.02).reshape(N, K))
+    X, x = bf16_dev(oracle.normal(81, 1, M * K).reshape(M, K), dev)
+    b = oracle.normal(81, 3, N, 0.02)
+    r = oracle.normal(81, 4, M * N).reshape(M, N)
+    Y = torch.empty((M, N), dtype=torch.float32, device=dev)
+    _gemm(cbis, M, N, K, X, cbis.BF16, to_dev(codes, dev), cbis.FP8E4M3, Y, cbis.F32, bias=to_dev(b, dev),
+          w_scale=to_dev(sc, dev), gelu=gelu, residual=to_dev(r, dev) if res else None, workspace=True)
+    rows = np.unique(np.concatenate([_sample_rows(M, 40, N + K), [0, M - 1]]))
+    w = oracle.e4m3_table()[codes].astype(np.float64) * sc.astype(np.float64)[:, None]
+    xr = x[rows].astype(np.float64)
+    ref = xr @ w.T + b
+    mag = np.abs(xr) @ np.abs(w).T + np.abs(b) + (np.abs(r[rows]) if res else 0)
+    tol = (K + 3) * 2.0 ** -23 * mag
+    if gelu:
+        from math import erf
+        ref = ref * 0.5 * (1 + np.vectorize(erf)(ref / np.sqrt(2)))
+        tol = 1.13 * tol + 1e-6 * (1 + np.abs(ref))
+    if res:
+        ref = ref + r[rows]
+    assert np.all(np.abs(Y.cpu().numpy()[rows] - ref) <= tol)
+
+
+@pytest.mark.parametrize("M,N,K", [(1216, 8000, 512), (300, 6007, 512), (65, 32000, 2048)])
+def test_gemm_argmax_fp8_tiles(cbis, oracle, dev, M, N, K):
+    """The greedy epilogue of the wave-specialised tiles with fp8 weights."""
+    test_gemm_argmax_matches_logits(cbis, oracle, dev, M, N, K, "fp8")
+
+
 def test_gemm_fp8_decode_every_code(cbis, oracle, dev):
     """Every OCP e4m3 code through the decode-sized (skinny) GEMM: row n of W
     holds code n at k = 0 and zeros elsewhere, X = e_0, scale 1, so
