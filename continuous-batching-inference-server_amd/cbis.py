@@ -105,6 +105,7 @@ KERNEL_SYMBOLS = {
     "cbis_paged_attention_static": (_I, [ctypes.POINTER(AttnDesc), _P]),
     "cbis_paged_attention_proj": (_I, [ctypes.POINTER(AttnDesc), ctypes.POINTER(GemmDesc), _P]),
     "cbis_paged_prefill_attention": (_I, [ctypes.POINTER(AttnDesc), _I, _P, _P]),
+    "cbis_paged_chunk_attention": (_I, [ctypes.POINTER(AttnDesc), _I, _P, _P]),
     "cbis_paged_attention_mixed": (_I, [ctypes.POINTER(AttnDesc), _I, _P, _P]),
     "cbis_embed": (_I, [_I, _I, _P, _P, _I, _P, _P, _I, _I, _P, _P]),
     "cbis_embed_from": (_I, [_I, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _P, _P, _P, _SZ, _P]),

@@ -889,6 +889,228 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
   }
 }
 
+// ---------------------------------------------------------------------------
+// Prefill over fp32 K/V on the fp32 MFMA.
+//
+// Workgroup: one tile of up to 16 consecutive query rows of a sequence and one
+// head, NW waves that take the sequence's 16-key pages round-robin and merge
+// their softmax states through LDS.  A page's K/V then serves 16 rows where the
+// decode kernel reads it once per row (a 512-row chunk after 4096 tokens, 8
+// heads: 4.6 GB a layer through the caches).  All arithmetic stays fp32, on
+// v_mfma_f32_16x16x4_f32, whose rate bounds the kernel (the K/V of a head come
+// from its XCD's L2: workgroups of one head share an XCD when n_heads is a
+// multiple of 8).
+//   S^T = K Q^T: lane (key = l % 16, quarter g = l / 16) holds K[key][8 g .. + 7]
+//     (two 16-byte loads), Q likewise; MFMA j takes dim 8 g + j of both.
+//   P^T stays where S^T was accumulated: lane (query, g) holds keys 4 g .. + 3.
+//   O^T = V^T P^T: MFMA (i, e) takes key 4 g + i and dim 2 (l % 16) + e, so a lane
+//     loads V[4 g + i][2 (l % 16) .. + 1], 8 bytes, a 128-byte row per 16 lanes.
+// Sixteen-row tiles give a 512-row chunk of 8 heads 256 workgroups; 32-row
+// tiles would halve the L2 reads and leave half the CUs idle.
+// ---------------------------------------------------------------------------
+struct ChunkArgs {
+  const int* tiles;  // [n_tiles][4]: first_row, n_valid, bt_row, first_pos
+  const void* q;
+  int64_t ldq;
+  int q_bf16;
+  const float* kpool;
+  const float* vpool;
+  int num_pages;
+  const int* bt;
+  int64_t bt_stride;
+  void* out;
+  int64_t ldo;
+  int out_bf16;
+  int n_heads;
+  int max_kv;
+  float qscale;
+};
+
+constexpr int kChunkRows = CBIS_CHUNK_TILE_ROWS;
+constexpr int kChunkWaves = 8;
+constexpr int kChunkRing = 3;  // pages per wave in registers: one computed, the others in flight
+static_assert(kChunkRows == 16, "16 x 16 MFMA tiles");
+
+// f over the four lanes that hold one query column (l, l ^ 16, l ^ 32, l ^ 48).
+__device__ inline float quarters_max(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+__device__ inline float quarters_sum(float v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
+__global__ __launch_bounds__(kChunkWaves * 64) void paged_chunk_f32_kernel(const ChunkArgs a) {
+  constexpr int NW = kChunkWaves, R = kChunkRing;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, qr = lane >> 4;
+  const int head = blockIdx.x % a.n_heads, tile = blockIdx.x / a.n_heads;
+  typedef const __attribute__((address_space(4))) int cint_t;
+  cint_t* td = (cint_t*)(a.tiles + (int64_t)4 * tile);
+  const int row0 = td[0], nvalid = min(td[1], kChunkRows), pos0 = td[3];
+  cint_t* bt = (cint_t*)(a.bt + (int64_t)td[2] * a.bt_stride);
+  const int D = a.n_heads * kHD;
+  const int kv_end = min(pos0 + nvalid, a.max_kv);  // keys [0, kv_end) needed by the tile
+  if (nvalid <= 0 || kv_end <= 0) return;
+
+  // Rows past the tile's end repeat its last row (computed, never stored).
+  const int qi = min(c, nvalid - 1), qpos = pos0 + qi;
+  float q[8];
+  if (a.q_bf16) {
+    const uint16_t* qp = (const uint16_t*)a.q + (int64_t)(row0 + qi) * a.ldq + head * kHD + 8 * qr;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = bf16_to_f32(qp[e]) * a.qscale;
+  } else {
+    const float* qp = (const float*)a.q + (int64_t)(row0 + qi) * a.ldq + head * kHD + 8 * qr;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = qp[e] * a.qscale;
+  }
+
+  // o[e][i]: dim 2 (4 qr + i) + e of query c; l: this lane's share of the
+  // probability sum (its own keys); m: the column's softmax reference.
+  f32x4_t o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  float l = 0.f, m = -INFINITY;
+
+  struct KV {
+    float4 k0, k1;
+    float2 v[4];
+  };
+  const int n_pages = (kv_end + kPS - 1) / kPS;
+  // Loads of page p: keys past kv_end read key kv_end - 1 (in bounds, masked).
+  auto load = [&](int p, KV& r) {
+    const int pc = min(p, n_pages - 1);
+    const int last = min(kPS, kv_end - pc * kPS) - 1;  // last key of the page that is read
+    const int64_t base = (int64_t)min(max(bt[pc], 0), a.num_pages - 1) * kPS * D + head * kHD;
+    const float* kp = a.kpool + base + min(c, last) * D + 8 * qr;
+    r.k0 = *(const float4*)kp;
+    r.k1 = *(const float4*)(kp + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.v[i] = *(const float2*)(a.vpool + base + min(4 * qr + i, last) * D + 2 * c);
+  };
+  auto compute = [&](int p, const KV& r) {
+    const float nm = m == -INFINITY ? 0.f : -m;
+    f32x4_t s = {nm, nm, nm, nm};  // scores come out relative to m
+    const float kk[8] = {r.k0.x, r.k0.y, r.k0.z, r.k0.w, r.k1.x, r.k1.y, r.k1.z, r.k1.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[j], q[j], s, 0, 0, 0);
+    const bool diag = p * kPS + kPS - 1 > pos0 || p * kPS + kPS > kv_end;  // uniform: some key masked for some row
+    if (diag) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int kj = p * kPS + 4 * qr + i;
+        if (kj > qpos || kj >= kv_end) s[i] = -INFINITY;
+      }
+    }
+    // m is raised only when a score exceeds it by more than kLazyRescale (or
+    // on a column's first unmasked key), so p = 2^s <= 2^8.
+    const float smax = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+    const float thr = m == -INFINITY ? -INFINITY : kLazyRescale;
+    if (__builtin_amdgcn_ballot_w64(smax > thr) != 0) {
+      const float cmax = quarters_max(smax), cur = m == -INFINITY ? 0.f : m;
+      const bool up = cmax > thr;
+      const float mn = up ? fmaxf(m, cmax + cur) : m;
+      const float corr = up && m != -INFINITY ? fast_exp2(m - mn) : 1.f;
+      const float d = up ? mn - cur : 0.f;
+      l *= corr;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[i] -= d;
+        o[0][i] *= corr;
+        o[1][i] *= corr;
+      }
+      m = mn;
+    }
+    float pr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      pr[i] = fast_exp2(s[i]);
+      l += pr[i];
+    }
+    float2 v[4] = {r.v[0], r.v[1], r.v[2], r.v[3]};
+    if (diag) {
+      // A key that some rows of the tile do not attend to must not reach
+      // them through 0 * inf: non-finite V values stay out of the product and
+      // are added to the rows that do attend, one key at a time.
+      bool bad = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool bx = !(fabsf(v[i].x) < INFINITY), by = !(fabsf(v[i].y) < INFINITY);
+        bad = bad || bx || by;
+        v[i].x = bx ? 0.f : v[i].x;
+        v[i].y = by ? 0.f : v[i].y;
+      }
+      if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+        for (int k = 0; k < kPS; ++k) {
+          const int src = (k >> 2) * 16;
+          const int i = k & 3;
+          const float mine = i == 0 ? pr[0] : i == 1 ? pr[1] : i == 2 ? pr[2] : pr[3];
+          const float pk = __shfl(mine, src + c, 64);
+          const float2 own = i == 0 ? r.v[0] : i == 1 ? r.v[1] : i == 2 ? r.v[2] : r.v[3];
+          const int kj = p * kPS + k;
+          const bool use = kj <= qpos && kj < kv_end;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const float vx = __shfl(own.x, src + 4 * qr + t, 64), vy = __shfl(own.y, src + 4 * qr + t, 64);
+            if (use && !(fabsf(vx) < INFINITY)) o[0][t] += pk * vx;
+            if (use && !(fabsf(vy) < INFINITY)) o[1][t] += pk * vy;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i].x, pr[i], o[0], 0, 0, 0);
+      o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i].y, pr[i], o[1], 0, 0, 0);
+    }
+  };
+
+  // This wave's pages wave, wave + NW, ... through a ring of R register slots.
+  KV ring[R];
+#pragma unroll
+  for (int u = 0; u < R - 1; ++u) load(wave + NW * u, ring[u]);
+  for (int p0 = wave; p0 < n_pages; p0 += NW * R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int p = p0 + NW * u;
+      load(p + NW * (R - 1), ring[(u + R - 1) % R]);
+      if (p < n_pages) compute(p, ring[u]);
+    }
+  }
+
+  // Merge the waves per query column; a wave without pages (or whose keys are
+  // all masked for the column) has m = -inf and contributes nothing.
+  __shared__ float sm[NW][16], sl[NW][16], so[NW][16][kHD + 1];
+  l = quarters_sum(l);
+  if (qr == 0) {
+    sm[wave][c] = m;
+    sl[wave][c] = l;
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) so[wave][c][2 * (4 * qr + i) + e] = o[e][i];
+  __syncthreads();
+  static_assert(NW * 64 == 16 * kHD, "one thread per output");
+  const int row = threadIdx.x / kHD, d = threadIdx.x % kHD;
+  if (row >= nvalid) return;
+  float M = sm[0][row];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) M = fmaxf(M, sm[w][row]);
+  float L = 0.f, O = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const float f = sm[w][row] == -INFINITY ? 0.f : fast_exp2(sm[w][row] - M);
+    L += sl[w][row] * f;
+    O += so[w][row][d] * f;
+  }
+  const float res = O / L;
+  const int64_t at = (int64_t)(row0 + row) * a.ldo + head * kHD + d;
+  if (a.out_bf16) ((uint16_t*)a.out)[at] = f32_to_bf16(res);
+  else ((float*)a.out)[at] = res;
+}
+
 int resolve_split(const cbis_attn_desc* d, int hblocks, int* n_splits) {
   int split = d->split_tokens;
   const int max_kv = std::max(1, d->max_kv_len);
@@ -1207,6 +1429,37 @@ int cbis_paged_prefill_attention(const cbis_attn_desc* d, int n_tiles, const int
   rc = check_tiles(d, n_tiles, tiles, "cbis_paged_prefill_attention");
   if (rc || n_tiles == 0) return rc;
   return prefill_launch(d, n_tiles, tiles, (hipStream_t)stream, nullptr, 0, "cbis_paged_prefill_attention");
+}
+
+int cbis_paged_chunk_attention(const cbis_attn_desc* d, int n_tiles, const int* tiles, cbis_stream_t stream) {
+  const char* who = "cbis_paged_chunk_attention";
+  const int rc = validate(d, who);
+  if (rc) return rc;
+  CBIS_REQUIRE(n_tiles >= 0, CBIS_ERR_INVALID, "%s: n_tiles < 0", who);
+  if (n_tiles == 0) return CBIS_OK;
+  CBIS_REQUIRE(d->kv_dtype == CBIS_F32, CBIS_ERR_UNSUPPORTED, "%s: needs fp32 K/V", who);
+  CBIS_REQUIRE(tiles && ((uintptr_t)tiles & 15u) == 0 && d->tile_pages == 0, CBIS_ERR_INVALID,
+               "%s: tiles must be a 16-byte aligned device array [n_tiles][4]", who);
+  ChunkArgs a;
+  a.tiles = tiles;
+  a.q = d->q;
+  a.ldq = d->ldq;
+  a.q_bf16 = d->q_dtype == CBIS_BF16;
+  a.kpool = (const float*)d->k_pool;
+  a.vpool = (const float*)d->v_pool;
+  a.num_pages = d->num_pages;
+  a.bt = d->block_table;
+  a.bt_stride = d->bt_stride;
+  a.out = d->out;
+  a.ldo = d->ldo;
+  a.out_bf16 = d->out_dtype == CBIS_BF16;
+  a.n_heads = d->n_heads;
+  a.max_kv = (int)std::min<int64_t>(d->bt_stride * kPS, 1 << 30);
+  a.qscale = kLog2e / sqrtf((float)kHD);
+  const int64_t grid = (int64_t)n_tiles * d->n_heads;
+  CBIS_REQUIRE(grid < (1LL << 31), CBIS_ERR_UNSUPPORTED, "%s: grid too large", who);
+  paged_chunk_f32_kernel<<<(unsigned)grid, kChunkWaves * 64, 0, (hipStream_t)stream>>>(a);
+  return check_launch(who);
 }
 
 int cbis_paged_attention_mixed(const cbis_attn_desc* d, int n_tiles, const int* tiles, cbis_stream_t stream) {

@@ -150,8 +150,14 @@ void TransformerRunner::prepare(int b, const int* tok, const int* pos, const int
     rowbt[i] = cur_idx;
   }
   // Rows: runs of consecutive positions of one sequence go to the MFMA
-  // prefill kernel (bf16 K/V), everything else to the split-KV decode kernel.
-  const bool prefill_ok = cfg_.kv_dtype == CBIS_BF16;
+  // prefill kernel of the K/V dtype, everything else to the split-KV decode
+  // kernel.  Small fp32 steps that can take the fused attention +
+  // out-projection launch keep all their rows in it.
+  const bool bf16_kv = cfg_.kv_dtype == CBIS_BF16;
+  int top_pos = 0;
+  for (int i = 0; i < M; ++i) top_pos = std::max(top_pos, pos[i]);
+  const bool prefill_ok = bf16_kv || !(fuse_decode_ && attn_proj_ok_ && M <= 64 && top_pos < 768);
+  const int tile_rows = bf16_kv ? kTileRows : CBIS_CHUNK_TILE_ROWS, tile_ints = bf16_kv ? kTileInts : 4;
   std::vector<int> drows, tiles;
   int max_kv = 1;
   int64_t sum_kv = 0;
@@ -160,9 +166,10 @@ void TransformerRunner::prepare(int b, const int* tok, const int* pos, const int
     while (j < M && seq[j] == seq[i] && pos[j] == pos[j - 1] + 1) ++j;
     if (prefill_ok && j - i >= kMinPrefillRun) {
       const std::vector<int>& pg = cache_.pages(seq[i]);
-      for (int r = i; r < j; r += kTileRows) {
-        const int nv = std::min(kTileRows, j - r);
+      for (int r = i; r < j; r += tile_rows) {
+        const int nv = std::min(tile_rows, j - r);
         tiles.insert(tiles.end(), {r, nv, rowbt[r], pos[r]});
+        if (!bf16_kv) continue;
         // The pages of the tile's first key blocks (tile_pages = 8): page
         // min(16 k, kv_end - 1) / 16, kv_end = pos[r] + nv (within the
         // sequence's pages, so within the step's block-table width).
@@ -183,23 +190,23 @@ void TransformerRunner::prepare(int b, const int* tok, const int* pos, const int
   // tail.
   std::stable_sort(drows.begin(), drows.end(), [&](int x, int y) { return pos[x] > pos[y]; });
   // Likewise the prefill tiles, by their last key (a tile's work grows with
-  // it), with the lighter half reversed: when the grid fits one round of
-  // resident workgroups, workgroup w and w + grid/2 share a CU, so the
+  // it); for bf16 K/V with the lighter half reversed: when the grid fits one
+  // round of resident workgroups, workgroup w and w + grid/2 share a CU, so the
   // heaviest tile shares its CU with the lightest (config 4: 25.5 -> 23.3 us).
   {
-    const int nt = (int)tiles.size() / kTileInts;
+    const int nt = (int)tiles.size() / tile_ints;
     std::vector<int> order(nt);
     for (int t = 0; t < nt; ++t) order[t] = t;
-    auto last_key = [&](int t) { return tiles[kTileInts * t + 3] + tiles[kTileInts * t + 1]; };
+    auto last_key = [&](int t) { return tiles[tile_ints * t + 3] + tiles[tile_ints * t + 1]; };
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return last_key(x) > last_key(y); });
-    std::reverse(order.begin() + nt / 2, order.end());
+    if (bf16_kv) std::reverse(order.begin() + nt / 2, order.end());
     std::vector<int> sorted(tiles.size());
-    for (int t = 0; t < nt; ++t) std::copy_n(&tiles[kTileInts * order[t]], kTileInts, &sorted[kTileInts * t]);
+    for (int t = 0; t < nt; ++t) std::copy_n(&tiles[tile_ints * order[t]], tile_ints, &sorted[tile_ints * t]);
     tiles.swap(sorted);
   }
   M_ = M;
   n_decode_ = (int)drows.size();
-  n_tiles_ = (int)tiles.size() / kTileInts;
+  n_tiles_ = (int)tiles.size() / tile_ints;
   n_seqs_ = (int)seqs.size();
   bt_width_ = width;
   max_kv_ = (max_kv + 255) / 256 * 256;  // coarse, so steps share split shapes (and graphs)
@@ -332,7 +339,8 @@ void TransformerRunner::enqueue_forward(int b, bool greedy, bool from_prev) {
   a.split_tokens = split_tokens_;
   a.workspace = d_ws_;
   a.workspace_bytes = ws_bytes_;
-  a.tile_pages = 8;
+  const bool bf16_kv = cfg_.kv_dtype == CBIS_BF16;
+  a.tile_pages = bf16_kv ? 8 : 0;
 
   // LayerNorms that follow a residual GEMM (ln2 after the out-projection,
   // the next layer's ln1 or ln_f after fc2) run with it (cbis_gemm_layernorm:
@@ -377,8 +385,10 @@ void TransformerRunner::enqueue_forward(int b, bool greedy, bool from_prev) {
       cbis_check(cbis_paged_attention_proj(&a, &g, s), "attention + out-proj");
     } else {
       // Single rows on the split-KV decode kernel, runs of rows on the MFMA
-      // prefill kernel (whose launch also merges the decode rows' splits).
-      cbis_check(cbis_paged_attention_mixed(&a, n_tiles_, d_tiles_, s), "attention");
+      // prefill kernel (for bf16 K/V its launch also merges the decode rows'
+      // splits).
+      cbis_check(cbis_paged_attention_mixed(&a, bf16_kv ? n_tiles_ : 0, d_tiles_, s), "attention");
+      if (!bf16_kv) cbis_check(cbis_paged_chunk_attention(&a, n_tiles_, d_tiles_, s), "chunk attention");
       if (ln_pro) cbis_check(cbis_gemm(&g, s), "out-proj gemm");
       else cbis_check(cbis_gemm_layernorm(&g, L.ln2_w, L.ln2_b, 1e-5f, act, d_xn_, D, s), "out-proj gemm + ln2");
     }

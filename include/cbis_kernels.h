@@ -275,6 +275,18 @@ int cbis_paged_attention_static(const cbis_attn_desc* d, cbis_stream_t stream);
 int cbis_paged_prefill_attention(const cbis_attn_desc* d, int n_tiles, const int* tiles,
                                  cbis_stream_t stream);
 
+/* Rows per tile of cbis_paged_chunk_attention, at most. */
+#define CBIS_CHUNK_TILE_ROWS 16
+
+/* Prefill attention over fp32 K/V (the fp32 MFMA; every operand, probability
+ * and sum in fp32) for query tiles of <= CBIS_CHUNK_TILE_ROWS consecutive rows
+ * of one sequence: tiles as for cbis_paged_prefill_attention with
+ * d->tile_pages = 0.  A row of a tile past CBIS_CHUNK_TILE_ROWS is not
+ * computed.  Q and out fp32 or bf16, head_dim 32, page_size 16, any n_heads;
+ * d->rows / row_bt / row_pos / max_kv_len / split_tokens / workspace are
+ * ignored. */
+int cbis_paged_chunk_attention(const cbis_attn_desc* d, int n_tiles, const int* tiles, cbis_stream_t stream);
+
 /* A step's attention in two launches: cbis_paged_attention over d's rows (the
  * single decode rows) then cbis_paged_prefill_attention over the tiles, with
  * the decode rows' split merge run inside the prefill launch instead of a

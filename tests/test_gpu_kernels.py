@@ -1517,6 +1517,106 @@ def test_prefill_attention_lazy_rescale(cbis, oracle, dev, mode):
     assert err_head < LOWP_TOL * 2
 
 
+@pytest.mark.parametrize("H", [1, 8, 12])
+@pytest.mark.parametrize("qdt,odt", [("f32", "f32"), ("bf16", "bf16")])
+def test_chunk_attention_f32(cbis, oracle, dev, H, qdt, odt):
+    """cbis_paged_chunk_attention (fp32 K/V tiles) against the fp64 oracle:
+    tiles of 1, 15 and 16 rows, fresh and after cached tokens, first position
+    and kv end either side of a page boundary, a single key, fewer pages than
+    waves and many more, and queries large enough to raise the softmax
+    reference after the first page.  The slots past each sequence's end hold
+    NaN and must not reach a row.  Rows of no tile stay untouched."""
+    import torch
+    seqs = [(0, 1), (0, 16), (0, 33), (15, 2), (16, 15), (31, 17), (100, 40), (900, 47), (5000, 31)]  # cached, rows
+    D, g = H * 32, rng(7 + H)
+    kv = [a + n for a, n in seqs]
+    npages = [-(-n // 16) for n in kv]
+    P = sum(npages) + 3
+    perm = g.permutation(P).astype(np.int32)
+    bt = np.zeros((len(seqs), max(npages)), np.int32)
+    at = 0
+    kp = g.standard_normal((P, 16, H, 32)).astype(np.float32)
+    vp = g.standard_normal((P, 16, H, 32)).astype(np.float32)
+    tiles, pos, row_seq, row = [], [], [], 0
+    for s, (cached, n) in enumerate(seqs):
+        bt[s, : npages[s]] = perm[at: at + npages[s]]
+        at += npages[s]
+        if kv[s] % 16:
+            kp[bt[s, npages[s] - 1], kv[s] % 16:] = np.nan
+            vp[bt[s, npages[s] - 1], kv[s] % 16:] = np.nan
+        for r in range(0, n, 16):
+            tiles.append([row + r, min(16, n - r), s, cached + r])
+        pos += range(cached, cached + n)
+        row_seq += [s] * n
+        row += n
+    M = row
+    q = g.standard_normal((M + 2, D)).astype(np.float32) * np.float32(4.0)
+    Q = bf16_dev(q, dev) if qdt == "bf16" else (to_dev(q, dev), q)
+    out = torch.full((M + 2, D), 7.0, dtype=torch.float32 if odt == "f32" else torch.bfloat16, device=dev)
+    BT, T = to_dev(bt, dev), to_dev(np.array(tiles, np.int32), dev)
+    KP, VP = to_dev(kp, dev), to_dev(vp, dev)
+    d = _attn_desc(cbis, 0, H, Q[0], KP, VP, P, BT, bt.shape[1], None, out, cbis.F32,
+                   q_dtype=cbis.F32 if qdt == "f32" else cbis.BF16, out_dtype=cbis.F32 if odt == "f32" else cbis.BF16)
+    cbis.check(cbis.kernels().cbis_paged_chunk_attention(ctypes.byref(d), len(tiles), ptr(T), stream()))
+    sync()
+    ref = oracle.paged_attention(Q[1][:M], np.nan_to_num(kp), np.nan_to_num(vp), bt[row_seq], np.array(pos, np.int32),
+                                 H, 32, 16)
+    got = out.float().cpu().numpy()
+    assert np.abs(got[:M] - ref).max() < (FP32_TOL if odt == "f32" else 2e-2)
+    assert (got[M:] == 7.0).all()
+
+
+def test_chunk_attention_f32_matches_decode_rows(cbis, dev):
+    """Rows do not depend on later rows of their tile: with inf and NaN in the
+    K/V of one position, the rows before it equal the decode kernel's (to fp32
+    rounding) and the rows from it on are not finite in the same places."""
+    import torch
+    H, n, cached = 8, 48, 20
+    g = rng(3)
+    P = -(-(cached + n) // 16)
+    k = g.standard_normal((P, 16, H, 32)).astype(np.float32)
+    v = g.standard_normal((P, 16, H, 32)).astype(np.float32)
+    for key, arr, val in ((30, v, np.inf), (41, v, np.nan), (52, k, np.nan), (63, v, -np.inf)):
+        arr[key // 16, key % 16, key % H, key % 32] = val
+    bt = np.arange(P, dtype=np.int32)[None]
+    q = g.standard_normal((n, H * 32)).astype(np.float32)
+    Q, K, V, BT = to_dev(q, dev), to_dev(k, dev), to_dev(v, dev), to_dev(bt, dev)
+    POS = to_dev(np.arange(cached, cached + n, dtype=np.int32), dev)
+    RB = to_dev(np.zeros(n, np.int32), dev)
+    T = to_dev(np.array([[r, 16, 0, cached + r] for r in range(0, n, 16)], np.int32), dev)
+    outs = []
+    for chunk in (True, False):
+        out = torch.empty((n, H * 32), dtype=torch.float32, device=dev)
+        d = _attn_desc(cbis, 0 if chunk else n, H, Q, K, V, P, BT, P, POS, out, cbis.F32, row_bt=RB)
+        if chunk:
+            cbis.check(cbis.kernels().cbis_paged_chunk_attention(ctypes.byref(d), 3, ptr(T), stream()))
+        else:
+            cbis.check(cbis.kernels().cbis_paged_attention(ctypes.byref(d), stream()))
+        sync()
+        outs.append(out.cpu().numpy())
+    fin = np.isfinite(outs[1])
+    assert fin[:10].all() and not fin[10:].all()
+    assert np.array_equal(np.isfinite(outs[0]), fin)
+    assert np.abs(outs[0][fin] - outs[1][fin]).max() < 1e-5
+
+
+def test_chunk_attention_rejects_unsupported(cbis, dev):
+    import torch
+    x = torch.zeros(1024, dtype=torch.float32, device=dev)
+    i = torch.zeros(64, dtype=torch.int32, device=dev)
+    K = cbis.kernels()
+    d = _attn_desc(cbis, 0, 1, x, x, x, 1, i, 1, i, x, cbis.BF16)
+    assert K.cbis_paged_chunk_attention(ctypes.byref(d), 1, ptr(i), stream()) == 2
+    d.kv_dtype = cbis.F32
+    assert K.cbis_paged_chunk_attention(ctypes.byref(d), -1, ptr(i), stream()) == 1
+    assert K.cbis_paged_chunk_attention(ctypes.byref(d), 1, None, stream()) == 1
+    assert K.cbis_paged_chunk_attention(ctypes.byref(d), 1, ptr(i) + 4, stream()) == 1
+    d.tile_pages = 8
+    assert K.cbis_paged_chunk_attention(ctypes.byref(d), 1, ptr(i), stream()) == 1
+    assert K.cbis_paged_chunk_attention(ctypes.byref(d), 0, None, stream()) == 0
+    sync()
+
+
 @pytest.mark.parametrize("kv_dtype,H", [("f32", 12), ("f32", 4), ("bf16", 24), ("bf16", 8)])
 def test_decode_attention_any_head_count(cbis, oracle, dev, kv_dtype, H):
     """Head counts that do not fill the last 1 KiB head block (8 fp32 or 16
