@@ -168,6 +168,48 @@ __device__ inline float wave_max(float v) {
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// ---------------------------------------------------------------------------
+// Direct-to-LDS loads.
+// ---------------------------------------------------------------------------
+__device__ inline void lds_dma16(const void* gptr, uint32_t lds_addr) {
+  // M0 is reserved by the compiler (it never keeps a value there across
+  // ordinary code), so it is set right before the load that reads it.
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
+}
+
+// The same from a wave-uniform base plus a 32-bit byte offset per lane.
+__device__ inline void lds_dma16(const void* base, uint32_t offset, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_addr) : "memory");
+}
+
+template <int N>
+__device__ inline void wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Waits until a wave's loads of a tile have landed, with `younger` (< STAGES)
+// tiles of LPW loads each issued after it.
+template <int LPW, int STAGES>
+__device__ inline void wait_dma_tile(int younger) {
+  static_assert(STAGES >= 2 && STAGES <= 8 && LPW * (STAGES - 1) < 64, "vmcnt range");
+  if constexpr (STAGES > 7) { if (younger >= 7) { wait_vmcnt<7 * LPW>(); return; } }
+  if constexpr (STAGES > 6) { if (younger >= 6) { wait_vmcnt<6 * LPW>(); return; } }
+  if constexpr (STAGES > 5) { if (younger >= 5) { wait_vmcnt<5 * LPW>(); return; } }
+  if constexpr (STAGES > 4) { if (younger >= 4) { wait_vmcnt<4 * LPW>(); return; } }
+  if constexpr (STAGES > 3) { if (younger >= 3) { wait_vmcnt<3 * LPW>(); return; } }
+  if constexpr (STAGES > 2) { if (younger >= 2) { wait_vmcnt<2 * LPW>(); return; } }
+  if (younger >= 1) wait_vmcnt<LPW>();
+  else wait_vmcnt<0>();
+}
+
+// LDS image of a 128-byte tile row: 16-byte chunk c of row r sits in slot
+// c ^ ((r >> 1) & 7).  gfx950 serves a ds_read_b128 16 lanes (256 bytes, all
+// 64 banks) per cycle; the 16 lanes of a fragment load read one chunk of 16
+// consecutive rows, i.e. 8 even rows in bytes 0-127 and 8 odd rows in bytes
+// 128-255 of the 64 banks, each set in 8 distinct slots: no bank conflicts.
+__device__ inline int swz_slot(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
+
 // LayerNorm of one row held by a 256-thread workgroup: the row's float4
 // chunk i (columns 4 (64 i + lane) .. + 3) is v[i / 4] of wave i % 4, gamma /
 // beta likewise.  The statistics are formed per lane over chunks 0 .. nch - 1

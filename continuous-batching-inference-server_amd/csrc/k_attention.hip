@@ -897,16 +897,25 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
 // their softmax states through LDS.  A page's K/V then serves 16 rows where the
 // decode kernel reads it once per row (a 512-row chunk after 4096 tokens, 8
 // heads: 4.6 GB a layer through the caches).  All arithmetic stays fp32, on
-// v_mfma_f32_16x16x4_f32, whose rate bounds the kernel (the K/V of a head come
-// from its XCD's L2: workgroups of one head share an XCD when n_heads is a
-// multiple of 8).
-//   S^T = K Q^T: lane (key = l % 16, quarter g = l / 16) holds K[key][8 g .. + 7]
-//     (two 16-byte loads), Q likewise; MFMA j takes dim 8 g + j of both.
-//   P^T stays where S^T was accumulated: lane (query, g) holds keys 4 g .. + 3.
-//   O^T = V^T P^T: MFMA (i, e) takes key 4 g + i and dim 2 (l % 16) + e, so a lane
-//     loads V[4 g + i][2 (l % 16) .. + 1], 8 bytes, a 128-byte row per 16 lanes.
+// v_mfma_f32_16x16x4_f32.
+//
+// A head's 128 bytes of K or V per key come into a per-wave LDS ring with
+// direct-to-LDS loads, eight lanes to a key (one key per lane would touch 16
+// lines per load), from a scalar base per page and lane offsets that only the
+// sequence's last page changes.
+//   S^T = K Q^T: MFMA row r is key 4 (r % 4) + r / 4 of the page; lane
+//     (r = l % 16, quarter g = l / 16) holds dims 8 g .. + 7 of it, Q likewise;
+//     MFMA j takes dim 8 g + j of both.  K rows are swizzled (swz_slot).
+//   P^T stays where S^T was accumulated: lane (query, g) holds in element i row
+//     4 g + i, i.e. key 4 i + g.
+//   O^T = V^T P^T: MFMA (i, e) takes key 4 i + g and dim 2 (l % 16) + e: a lane
+//     reads V[4 i + g][2 (l % 16) .. + 1], the wave 512 consecutive bytes.
 // Sixteen-row tiles give a 512-row chunk of 8 heads 256 workgroups; 32-row
-// tiles would halve the L2 reads and leave half the CUs idle.
+// tiles would halve the L2 reads and leave half the CUs idle.  Workgroups of one
+// head share an XCD (and its L2) when n_heads is a multiple of 8.
+// Measured (512 rows after 4096 cached tokens, 8 heads, one layer): 320 us with a
+// decode workgroup per row, 32 with K/V loaded into the operand registers, 29.3
+// so; the MFMAs alone need 16 at 2.4 GHz.  16 waves per workgroup: the same.
 // ---------------------------------------------------------------------------
 struct ChunkArgs {
   const int* tiles;  // [n_tiles][4]: first_row, n_valid, bt_row, first_pos
@@ -928,7 +937,8 @@ struct ChunkArgs {
 
 constexpr int kChunkRows = CBIS_CHUNK_TILE_ROWS;
 constexpr int kChunkWaves = 8;
-constexpr int kChunkRing = 3;  // pages per wave in registers: one computed, the others in flight
+constexpr int kChunkRing = 2;   // pages per wave in LDS: one computed, one in flight (3 and 4 measured the same)
+constexpr int kChunkSlot = 4096;  // bytes of a page's K and V for one head
 static_assert(kChunkRows == 16, "16 x 16 MFMA tiles");
 
 // f over the four lanes that hold one query column (l, l ^ 16, l ^ 32, l ^ 48).
@@ -950,7 +960,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void paged_chunk_f32_kernel(const
   typedef const __attribute__((address_space(4))) int cint_t;
   cint_t* td = (cint_t*)(a.tiles + (int64_t)4 * tile);
   const int row0 = td[0], nvalid = min(td[1], kChunkRows), pos0 = td[3];
-  cint_t* bt = (cint_t*)(a.bt + (int64_t)td[2] * a.bt_stride);
+  const int* bt = a.bt + (int64_t)td[2] * a.bt_stride;
   const int D = a.n_heads * kHD;
   const int kv_end = min(pos0 + nvalid, a.max_kv);  // keys [0, kv_end) needed by the tile
   if (nvalid <= 0 || kv_end <= 0) return;
@@ -971,42 +981,71 @@ __global__ __launch_bounds__(kChunkWaves * 64) void paged_chunk_f32_kernel(const
   // o[e][i]: dim 2 (4 qr + i) + e of query c; l: this lane's share of the
   // probability sum (its own keys); m: the column's softmax reference.
   f32x4_t o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  float l = 0.f, m = -INFINITY;
+  float l = 0.f, m = -INFINITY, thr = -INFINITY;
+  f32x4_t negm = {0.f, 0.f, 0.f, 0.f};  // -m, or 0 while m = -inf: the score MFMAs' C operand
 
-  struct KV {
-    float4 k0, k1;
-    float2 v[4];
-  };
   const int n_pages = (kv_end + kPS - 1) / kPS;
-  // Loads of page p: keys past kv_end read key kv_end - 1 (in bounds, masked).
-  auto load = [&](int p, KV& r) {
-    const int pc = min(p, n_pages - 1);
-    const int last = min(kPS, kv_end - pc * kPS) - 1;  // last key of the page that is read
-    const int64_t base = (int64_t)min(max(bt[pc], 0), a.num_pages - 1) * kPS * D + head * kHD;
-    const float* kp = a.kpool + base + min(c, last) * D + 8 * qr;
-    r.k0 = *(const float4*)kp;
-    r.k1 = *(const float4*)(kp + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.v[i] = *(const float2*)(a.vpool + base + min(4 * qr + i, last) * D + 2 * c);
+  __shared__ __attribute__((aligned(1024))) uint8_t ring_all[NW * R * kChunkSlot];
+  uint8_t* const ring = ring_all + wave * (R * kChunkSlot);
+  const uint32_t ring_lds =
+      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring);
+  // This wave's pages are wave, wave + NW, ...: page i of them goes to slot
+  // i % R.  Keys past kv_end read key kv_end - 1 (in bounds, masked).  Lane l
+  // holds the id of page 64 b + l of them: a scalar load per page would make
+  // every LDS wait of the page before wait for it too (one counter).
+  const int mine = n_pages > wave ? (n_pages - wave + NW - 1) / NW : 0;
+  int ids = 0;
+  const int drow = lane >> 3;  // row of the DMA instruction's eight
+  // Byte offsets of this lane's 16 bytes from the head's slice of a page's
+  // first key, when key `last` is the last one that is read.
+  uint32_t kb0, kb1, vb0, vb1;
+  auto offsets = [&](int last) {
+    const uint32_t r0 = min(drow, last) * D * 4, r1 = min(drow + 8, last) * D * 4;
+    kb0 = r0 + swz_slot(drow, lane & 7) * 16;
+    kb1 = r1 + swz_slot(drow + 8, lane & 7) * 16;
+    vb0 = r0 + (lane & 7) * 16;
+    vb1 = r1 + (lane & 7) * 16;
   };
-  auto compute = [&](int p, const KV& r) {
-    const float nm = m == -INFINITY ? 0.f : -m;
-    f32x4_t s = {nm, nm, nm, nm};  // scores come out relative to m
-    const float kk[8] = {r.k0.x, r.k0.y, r.k0.z, r.k0.w, r.k1.x, r.k1.y, r.k1.z, r.k1.w};
+  offsets(kPS - 1);
+  auto issue = [&](int i) {
+    if ((i & 63) == 0) {
+      ids = bt[min(wave + NW * (i + lane), n_pages - 1)];
+      asm volatile("" : "+v"(ids));  // waited for here, not (with the ring's loads) at every page
+    }
+    const int id = __builtin_amdgcn_readlane(ids, i & 63);
+    const int left = kv_end - (wave + NW * i) * kPS;
+    if (left < kPS) offsets(left - 1);  // the sequence's last page: this wave's last
+    const int64_t base = (int64_t)min(max(id, 0), a.num_pages - 1) * kPS * D + head * kHD;
+    const uint32_t slot = ring_lds + (uint32_t)(i % R) * kChunkSlot;
+    lds_dma16(a.kpool + base, kb0, slot);
+    lds_dma16(a.kpool + base, kb1, slot + 1024);
+    lds_dma16(a.vpool + base, vb0, slot + 2048);
+    lds_dma16(a.vpool + base, vb1, slot + 3072);
+  };
+  const int krow = 4 * (c & 3) + (c >> 2);  // key of MFMA row c
+  const int kofs0 = krow * 128 + (swz_slot(krow, 2 * qr) << 4), kofs1 = krow * 128 + (swz_slot(krow, 2 * qr + 1) << 4);
+  auto compute = [&](int i) {
+    const int p = wave + NW * i;
+    const uint8_t* slot = ring + (i % R) * kChunkSlot;
+    const float4 k0 = *(const float4*)(slot + kofs0), k1 = *(const float4*)(slot + kofs1);
+    float2 v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = *(const float2*)(slot + 2048 + (4 * t + qr) * 128 + 8 * c);
+    f32x4_t s = negm;  // scores come out relative to m
+    const float kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
 #pragma unroll
     for (int j = 0; j < 8; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[j], q[j], s, 0, 0, 0);
     const bool diag = p * kPS + kPS - 1 > pos0 || p * kPS + kPS > kv_end;  // uniform: some key masked for some row
     if (diag) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int kj = p * kPS + 4 * qr + i;
+        const int kj = p * kPS + 4 * i + qr;
         if (kj > qpos || kj >= kv_end) s[i] = -INFINITY;
       }
     }
     // m is raised only when a score exceeds it by more than kLazyRescale (or
     // on a column's first unmasked key), so p = 2^s <= 2^8.
     const float smax = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    const float thr = m == -INFINITY ? -INFINITY : kLazyRescale;
     if (__builtin_amdgcn_ballot_w64(smax > thr) != 0) {
       const float cmax = quarters_max(smax), cur = m == -INFINITY ? 0.f : m;
       const bool up = cmax > thr;
@@ -1019,8 +1058,10 @@ __global__ __launch_bounds__(kChunkWaves * 64) void paged_chunk_f32_kernel(const
         s[i] -= d;
         o[0][i] *= corr;
         o[1][i] *= corr;
+        negm[i] = mn == -INFINITY ? 0.f : -mn;
       }
       m = mn;
+      thr = mn == -INFINITY ? -INFINITY : kLazyRescale;
     }
     float pr[4];
 #pragma unroll
@@ -1028,61 +1069,59 @@ __global__ __launch_bounds__(kChunkWaves * 64) void paged_chunk_f32_kernel(const
       pr[i] = fast_exp2(s[i]);
       l += pr[i];
     }
-    float2 v[4] = {r.v[0], r.v[1], r.v[2], r.v[3]};
     if (diag) {
       // A key that some rows of the tile do not attend to must not reach
       // them through 0 * inf: non-finite V values stay out of the product and
       // are added to the rows that do attend, one key at a time.
       bool bad = false;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bool bx = !(fabsf(v[i].x) < INFINITY), by = !(fabsf(v[i].y) < INFINITY);
+      for (int t = 0; t < 4; ++t) {
+        const bool bx = !(fabsf(v[t].x) < INFINITY), by = !(fabsf(v[t].y) < INFINITY);
         bad = bad || bx || by;
-        v[i].x = bx ? 0.f : v[i].x;
-        v[i].y = by ? 0.f : v[i].y;
+        v[t].x = bx ? 0.f : v[t].x;
+        v[t].y = by ? 0.f : v[t].y;
       }
       if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+#pragma unroll 1
         for (int k = 0; k < kPS; ++k) {
-          const int src = (k >> 2) * 16;
-          const int i = k & 3;
-          const float mine = i == 0 ? pr[0] : i == 1 ? pr[1] : i == 2 ? pr[2] : pr[3];
-          const float pk = __shfl(mine, src + c, 64);
-          const float2 own = i == 0 ? r.v[0] : i == 1 ? r.v[1] : i == 2 ? r.v[2] : r.v[3];
-          const int kj = p * kPS + k;
+          const int t = k >> 2, kj = p * kPS + k;
+          const float own = t == 0 ? pr[0] : t == 1 ? pr[1] : t == 2 ? pr[2] : pr[3];
+          const float pk = __shfl(own, (k & 3) * 16 + c, 64);
+          const float* vk = (const float*)(slot + 2048 + k * 128) + 8 * qr;  // dims 2 (4 qr + e), + 1
           const bool use = kj <= qpos && kj < kv_end;
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const float vx = __shfl(own.x, src + 4 * qr + t, 64), vy = __shfl(own.y, src + 4 * qr + t, 64);
-            if (use && !(fabsf(vx) < INFINITY)) o[0][t] += pk * vx;
-            if (use && !(fabsf(vy) < INFINITY)) o[1][t] += pk * vy;
+          for (int e = 0; e < 4; ++e) {
+            if (use && !(fabsf(vk[2 * e]) < INFINITY)) o[0][e] += pk * vk[2 * e];
+            if (use && !(fabsf(vk[2 * e + 1]) < INFINITY)) o[1][e] += pk * vk[2 * e + 1];
           }
         }
       }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i].x, pr[i], o[0], 0, 0, 0);
-      o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i].y, pr[i], o[1], 0, 0, 0);
+    for (int t = 0; t < 4; ++t) {
+      o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t].x, pr[t], o[0], 0, 0, 0);
+      o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t].y, pr[t], o[1], 0, 0, 0);
     }
   };
 
-  // This wave's pages wave, wave + NW, ... through a ring of R register slots.
-  KV ring[R];
-#pragma unroll
-  for (int u = 0; u < R - 1; ++u) load(wave + NW * u, ring[u]);
-  for (int p0 = wave; p0 < n_pages; p0 += NW * R) {
-#pragma unroll
-    for (int u = 0; u < R; ++u) {
-      const int p = p0 + NW * u;
-      load(p + NW * (R - 1), ring[(u + R - 1) % R]);
-      if (p < n_pages) compute(p, ring[u]);
-    }
+  for (int i = 0; i < R - 1; ++i)
+    if (i < mine) issue(i);
+  for (int i = 0; i < mine; ++i) {
+    // Slot (i - 1) % R: its reads fed MFMAs already issued, so they are done
+    // once the LDS counter is empty.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + R - 1 < mine) issue(i + R - 1);
+    wait_dma_tile<4, R>(min(mine - 1, i + R - 1) - i);
+    compute(i);
   }
 
   // Merge the waves per query column; a wave without pages (or whose keys are
   // all masked for the column) has m = -inf and contributes nothing.
-  __shared__ float sm[NW][16], sl[NW][16], so[NW][16][kHD + 1];
+  __shared__ float sm[NW][16], sl[NW][16];
+  auto so = (float(*)[16][kHD + 1])ring_all;  // [NW][16][kHD + 1], once every wave is done with its ring
+  static_assert(sizeof(float) * NW * 16 * (kHD + 1) <= sizeof(ring_all), "merge buffer");
   l = quarters_sum(l);
+  __syncthreads();
   if (qr == 0) {
     sm[wave][c] = m;
     sl[wave][c] = l;
@@ -1092,7 +1131,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void paged_chunk_f32_kernel(const
 #pragma unroll
     for (int i = 0; i < 4; ++i) so[wave][c][2 * (4 * qr + i) + e] = o[e][i];
   __syncthreads();
-  static_assert(NW * 64 == 16 * kHD, "one thread per output");
+  static_assert(NW * 64 >= 16 * kHD, "one thread per output");
   const int row = threadIdx.x / kHD, d = threadIdx.x % kHD;
   if (row >= nvalid) return;
   float M = sm[0][row];

@@ -265,12 +265,6 @@ __device__ inline int xcd_contiguous(int bid, int nwg) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (bid >> 3);
 }
 
-// LDS image of a 128-byte tile row: 16-byte chunk c of row r sits in slot
-// c ^ ((r >> 1) & 7).  gfx950 serves a ds_read_b128 16 lanes (256 bytes, all
-// 64 banks) per cycle; the 16 lanes of a fragment load read one chunk of 16
-// consecutive rows, i.e. 8 even rows in bytes 0-127 and 8 odd rows in bytes
-// 128-255 of the 64 banks, each set in 8 distinct slots: no bank conflicts.
-__device__ inline int swz_slot(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 __device__ inline int swz(int row, int chunk) { return row * 128 + (swz_slot(row, chunk) << 4); }
 
 template <int BM, int BN, int WM, int WN, int FM, int FN>
@@ -645,18 +639,6 @@ __global__ __launch_bounds__(256) void splitk_layernorm_kernel(const GemmArgs g,
 // vector-memory instruction is issued inside the main loop, so the vmcnt
 // immediates count exactly the DMA loads of the younger tiles.
 // ---------------------------------------------------------------------------
-__device__ inline void lds_dma16(const void* gptr, uint32_t lds_addr) {
-  // M0 is reserved by the compiler (it never keeps a value there across
-  // ordinary code), so it is set right before the load that reads it.
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
-}
-
-template <int N>
-__device__ inline void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // One stage of the ring: BM rows of X (128 bytes of K = 64 bf16 each), then BN
 // rows of W (64 K elements: 128 bytes of bf16, or 64 bytes of e4m3 codes, which
 // stay codes in LDS and are widened when a fragment is read).  A 1 KiB DMA
@@ -711,21 +693,6 @@ struct DmaTile {
     for (int j = 0; j < LB; ++j) lds_dma16(b[j] + kt * WROW, base + b_ofs(p, j));
   }
 };
-
-// Waits until a wave's loads of a K tile have landed, with `younger` (< STAGES)
-// tiles of LPW loads each issued after it.
-template <int LPW, int STAGES>
-__device__ inline void wait_dma_tile(int younger) {
-  static_assert(STAGES >= 2 && STAGES <= 8 && LPW * (STAGES - 1) < 64, "vmcnt range");
-  if constexpr (STAGES > 7) { if (younger >= 7) { wait_vmcnt<7 * LPW>(); return; } }
-  if constexpr (STAGES > 6) { if (younger >= 6) { wait_vmcnt<6 * LPW>(); return; } }
-  if constexpr (STAGES > 5) { if (younger >= 5) { wait_vmcnt<5 * LPW>(); return; } }
-  if constexpr (STAGES > 4) { if (younger >= 4) { wait_vmcnt<4 * LPW>(); return; } }
-  if constexpr (STAGES > 3) { if (younger >= 3) { wait_vmcnt<3 * LPW>(); return; } }
-  if constexpr (STAGES > 2) { if (younger >= 2) { wait_vmcnt<2 * LPW>(); return; } }
-  if (younger >= 1) wait_vmcnt<LPW>();
-  else wait_vmcnt<0>();
-}
 
 // The MFMA operands of one wave's (32 FM) x (32 FN) sub-tile for the 16-wide k
 // steps of a stage, double-buffered: load(ks + 1) may be issued before the
