@@ -151,12 +151,16 @@ void TransformerRunner::prepare(int b, const int* tok, const int* pos, const int
   }
   // Rows: runs of consecutive positions of one sequence go to the MFMA
   // prefill kernel of the K/V dtype, everything else to the split-KV decode
-  // kernel.  Small fp32 steps that can take the fused attention +
-  // out-projection launch keep all their rows in it.
+  // kernel.  Fp32 steps small enough for the fused attention +
+  // out-projection launch keep all their rows in it while their keys are few:
+  // that saves a launch per layer, and re-reading the keys for every row costs
+  // more than that from about 200 keys on (device time of the 4-layer step, all
+  // rows fused / in tiles: 4 x 16 rows at kv 32 247 / 270 us, 64 rows at kv 64 255 /
+  // 270 and at kv 256 279 / 274, 9 rows at kv 32 112 / 112 and at kv 256 149 / 116).
   const bool bf16_kv = cfg_.kv_dtype == CBIS_BF16;
   int top_pos = 0;
   for (int i = 0; i < M; ++i) top_pos = std::max(top_pos, pos[i]);
-  const bool prefill_ok = bf16_kv || !(fuse_decode_ && attn_proj_ok_ && M <= 64 && top_pos < 768);
+  const bool prefill_ok = bf16_kv || !(fuse_decode_ && attn_proj_ok_ && M <= 64 && top_pos < 128);
   const int tile_rows = bf16_kv ? kTileRows : CBIS_CHUNK_TILE_ROWS, tile_ints = bf16_kv ? kTileInts : 4;
   std::vector<int> drows, tiles;
   int max_kv = 1;
