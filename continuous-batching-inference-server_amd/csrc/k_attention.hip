@@ -520,28 +520,28 @@ struct PrefillArgs {
   float qscale;  // log2(e) / sqrt(head_dim), folded into Q before its bf16 rounding
 };
 
-// Workgroup: one tile of up to 64 query rows x HPW adjacent heads, NWH waves
-// per head.  A head's waves take its 32-key blocks round-robin (block b goes to
-// wave b % NWH) and merge their softmax states through LDS at the end.  Each
-// wave runs the tile's rows as kQG groups of 32 query columns against every key
-// block it loads, so a K/V block read from the pages serves 64 queries.
-//
-// K/V come into an LDS ring with direct-to-LDS loads in whole cache lines: the
-// two heads of a workgroup are 128 consecutive bytes of a token, and the two
-// waves that work on one key block (one per head) share its ring slot, one
-// loading K and the other V.  The kernel's long contexts are bound by the L2
-// requests (89% of them hit): with a key per lane in the operand layout, or with
-// a 64-byte head slice per wave, each line is asked for twice or more (one
-// layer, 512 rows after 16384 tokens, 64 heads: 198 us so, 149 with 64-byte DMA
-// rows, of which the loads alone took 144 and the arithmetic alone 109).
+// Workgroup: one tile of up to 64 query rows x HPW adjacent heads,
+// kPrefillWaves waves per head.  A head's waves take its 32-key blocks
+// round-robin (block b goes to wave b % kPrefillWaves) and merge their
+// softmax states through LDS at the end.  Each wave runs the tile's rows as
+// kQG groups of 32 query columns against every key block it loads, so a K/V
+// block read from the pages serves 64 queries.  A key's head_dim slice is
+// 64 bytes, so adjacent heads of one workgroup read the same 128-byte lines
+// at about the same time.  Measured on config 4's two 512-row chunks (one
+// layer, isolated): 16.3 us.  Slower: four waves per head (23.1 with one head
+// per workgroup, 24.9 with two), a tile pair per workgroup whose waves take
+// equal contiguous shares of both tiles' blocks (20.1), four waves per head
+// on the long tiles only (20.8 - 24.6: the workgroups' pairing on the CUs is
+// lost), deeper K/V rings (17.4 with 3 blocks, 18.8 with 4).
+constexpr int kPrefillWaves = 2;  // waves per head
 constexpr int kQG = 2;            // 32-query groups per tile
 static_assert(32 * kQG == CBIS_PREFILL_TILE_ROWS, "prefill tile rows");
-constexpr int kPrefillRing = 3;  // K/V blocks per key-block lane in LDS: one computed, the others in flight
+// K/V blocks per wave's register ring: one block in flight while one is
+// computed.
+constexpr int kPrefillRing = 2;
 // Exponent headroom of the lazy softmax rescale (log2 units): a score may
 // exceed the largest one seen when its reference was set by up to this much.
 constexpr float kLazyRescale = 8.f;
-// The bf16 kernel's reference lies this far above that score, so p < 2.
-constexpr float kLazyLead = kLazyRescale - 1.f;
 
 // The two 32-lane halves of v exchanged: each lane gets f(v, v of lane ^ 32)
 // through v_permlane32_swap (no LDS round trip).
@@ -556,14 +556,370 @@ typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 // Workgroups from prefill_blocks on run the decode rows' split merge
 // (decode_merge over merge_rows rows) instead: the merge then shares the
 // prefill launch, which is independent of it, in place of a launch of its own.
-template <int HPW, int NWH>
-__global__ __launch_bounds__(HPW * NWH * 64, 2) void paged_prefill_kernel(const PrefillArgs a, const DecodeArgs merge,
-                                                                          int merge_rows, unsigned prefill_blocks) {
+template <int HPW>
+__global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_kernel(const PrefillArgs a,
+                                                                               const DecodeArgs merge, int merge_rows,
+                                                                               unsigned prefill_blocks) {
   if (blockIdx.x >= prefill_blocks) {
     decode_merge(merge, merge_rows, (int64_t)(blockIdx.x - prefill_blocks) * blockDim.x + threadIdx.x);
     return;
   }
+  const int lane = threadIdx.x & 63;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: block tests and page ids per wave
+  const int wave = wave_id % kPrefillWaves;  // key-block lane of this head
+  const int hsub = wave_id / kPrefillWaves;
+  const int n_hg = a.n_heads / HPW;
+  const int tile = blockIdx.x / n_hg;
+  const int head = (blockIdx.x % n_hg) * HPW + hsub;
+  // The tile descriptor is the same for the whole workgroup: read it into
+  // scalar registers, so the tests on it (the causal-mask test per block)
+  // compile to scalar branches rather than exec masking.
+  // The tile descriptor is the same for the whole workgroup and the page ids
+  // of a 32-key block the same for the whole wave: both are read through the
+  // constant address space, i.e. with scalar loads (shorter round trips than
+  // per-lane loads of one address, and no share of the K/V loads' counter),
+  // and the tests on them compile to scalar branches.
+  typedef const __attribute__((address_space(4))) int cint_t;
+  cint_t* td = (cint_t*)(a.tiles + (int64_t)a.tile_ints * tile);
+  const int row0 = td[0], nvalid = td[1], pos0 = td[3];
+  cint_t* bt = (cint_t*)(a.bt + (int64_t)td[2] * a.bt_stride);
+  const int D = a.n_heads * kHD;
+  const int col = lane & 31;  // query index within a group (B / C column)
+  const int half = lane >> 5;
+
+  // Q^T of group g as the B operand: lane holds q[32 g + col][half*8 + 0..7]
+  // (MFMA 0) and q[32 g + col][16 + half*8 + 0..7] (MFMA 1), bf16.  Rows past
+  // the tile's end repeat its last row (computed, never stored).
+  bf16x8_t qb0[kQG], qb1[kQG];
+  int qpos[kQG];
+#pragma unroll
+  for (int g = 0; g < kQG; ++g) {
+    const int qi = min(32 * g + col, nvalid - 1);
+    const int qr = row0 + qi;
+    qpos[g] = pos0 + qi;
+    float f[16];
+    if (a.q_bf16) {
+      const uint16_t* qp = (const uint16_t*)a.q + (int64_t)qr * a.ldq + head * kHD;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        f[e] = bf16_to_f32(qp[half * 8 + e]);
+        f[8 + e] = bf16_to_f32(qp[16 + half * 8 + e]);
+      }
+    } else {
+      const float* qp = (const float*)a.q + (int64_t)qr * a.ldq + head * kHD;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        f[e] = qp[half * 8 + e];
+        f[8 + e] = qp[16 + half * 8 + e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      qb0[g][e] = (short)f32_to_bf16(f[e] * a.qscale);
+      qb1[g][e] = (short)f32_to_bf16(f[8 + e] * a.qscale);
+    }
+  }
+  const int kv_end = min(pos0 + nvalid, a.max_kv);  // keys [0, kv_end) needed by the tile
+
+  // Per-wave V tile [key][dim]: 64-byte rows of four 16-byte chunks, chunk c
+  // of key row r in position c ^ ((r >> 2) & 3).  Unswizzled, the 16 lanes
+  // of a ds_write_b128 (keys 0..15, one chunk) hit 4 bank groups 4 times
+  // each; swizzled, 16 distinct groups.
+  __shared__ __attribute__((aligned(16))) uint8_t vt_all[HPW * kPrefillWaves][32 * kHD * 2];
+  uint8_t* const vt_w = vt_all[wave_id];
+  auto vpos = [](int key, int chunk) { return key * (kHD * 2) + ((chunk ^ ((key >> 2) & 3)) << 4); };
+  // Per query column: o (the P.V accumulator), lacc (every entry the
+  // column's sum of the bf16-rounded p: an MFMA of an all-ones A with P^T,
+  // beside the P.V MFMAs, in place of 16 adds and a lane exchange per block)
+  // and the softmax reference m (-inf until the column meets an unmasked
+  // key).  negm (every entry -m, or 0 while m = -inf) is the C operand of
+  // the score MFMA, so the scores come out relative to m and p = 2^s needs
+  // no subtraction per score.
+  f32x16_t o[kQG], lacc[kQG], negm[kQG];
+  float m[kQG];
+  bf16x8_t ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = (short)0x3F80;
+#pragma unroll
+  for (int g = 0; g < kQG; ++g) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[g][i] = lacc[g][i] = negm[g][i] = 0.f;
+    m[g] = -INFINITY;
+  }
+
+  // K rows for keys j0 + col in the A-operand layout (lane = key, dims
+  // half*8.. and 16 + half*8..) and this lane's half of the key's V row.
+  struct KV {
+    bf16x8_t k0, k1;
+    uint4 v0, v1;
+  };
+  // A block's 32 keys span two pages.  Each lane reads the page id of its
+  // own key (id_of) one block before that block's K/V loads (load_block):
+  // the id load then has a whole block of compute to land in, and waiting
+  // for it never waits for the K/V loads in flight.
+  // Page id of this lane's key j0 + col, clamped to kv_end - 1: keys j0 ..
+  // j0 + 15 lie on page min(j0, kv_end - 1) / 16, keys j0 + 16 .. j0 + 31 on
+  // page min(j0 + 16, kv_end - 1) / 16 (j0 is a multiple of 32).
+  // The ids are clamped to the pool here, in scalar registers.
+  auto id_of = [&](int j0) {
+    const unsigned last = (unsigned)(kv_end - 1);
+    const int pa = min(max(bt[min((unsigned)j0, last) / kPS], 0), a.num_pages - 1);
+    const int pb = min(max(bt[min((unsigned)j0 + 16u, last) / kPS], 0), a.num_pages - 1);
+    return col < 16 ? pa : pb;
+  };
+  // Element offset of this lane's key within its page, plus its head:
+  // (col % 16) * D + head * kHD for every block that ends before kv_end.
+  const int lane_off = (col & (kPS - 1)) * D + head * kHD;
+  const int64_t page_elems = (int64_t)kPS * D;
+  auto load_block = [&](int j0, int phys, KV& r) {
+    int off = lane_off;
+    if (j0 + 31 >= kv_end) off = (min(j0 + col, kv_end - 1) & (kPS - 1)) * D + head * kHD;
+    const int64_t slot = phys * page_elems + off;
+    r.k0 = *(const bf16x8_t*)(a.kpool + slot + half * 8);
+    r.k1 = *(const bf16x8_t*)(a.kpool + slot + 16 + half * 8);
+    const uint4* vs = (const uint4*)(a.vpool + slot + half * 16);
+    r.v0 = vs[0];
+    r.v1 = vs[1];
+  };
+  // ds_read_b64_tr_b16 reads in 16-lane groups: lane i of a group receives
+  // element i % 4 of the 8-byte rows addressed by lanes i / 4 + 4 e of the
+  // group, e = 0..3.  Lane (group gq, j) addresses key kr = 4 (gq / 2) + j / 4
+  // (+ 8, 16, 24), dims 16 (gq % 2) + 4 (j % 4) .. + 3, so lane (dim d, half h)
+  // receives V[4 h + e][d] (+ 8, 16, 24): the A-operand layout of V^T below.
+  const int kr = 4 * ((lane >> 4) >> 1) + ((lane & 15) >> 2);
+  const int dc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  // Byte offsets of the 8-byte rows read for keys kr + 8 m (m = 0..3) and of
+  // this lane's two V chunks (key col, dims 16 half .. + 15).
+  int vrd[4];
+#pragma unroll
+  for (int mm = 0; mm < 4; ++mm) vrd[mm] = vpos(kr + 8 * mm, dc >> 3) + (dc & 7) * 2;
+  const int vwr0 = vpos(col, 2 * half), vwr1 = vpos(col, 2 * half + 1);
+  auto vt_read = [&](int mm) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_short4_t*)(__attribute__((address_space(3))) void*)(vt_w + vrd[mm]));
+  };
+  auto compute_block = [&](int j0, const KV& r) {
+    *(uint4*)(vt_w + vwr0) = r.v0;  // this lane's key, dims 16 half .. + 7
+    *(uint4*)(vt_w + vwr1) = r.v1;  // and + 8 .. + 15
+    bf16x8_t pb0[kQG], pb1[kQG];
+    // Both groups' scores first (no branch between their MFMAs), then one
+    // uniform mask test and one uniform rescale test for the block.
+    // s[g][i]: key j0 + 8*(i/4) + 4*half + (i%4), query 32 g + col, in log2
+    // units relative to m: q.k * log2(e)/sqrt(hd) - m (the scale is folded
+    // into Q).  Only blocks reaching past the tile's first query position or
+    // past kv_end need the causal mask.
+    f32x16_t s[kQG];
+#pragma unroll
+    for (int g = 0; g < kQG; ++g) {
+      s[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(r.k0, qb0[g], negm[g], 0, 0, 0);
+      s[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(r.k1, qb1[g], s[g], 0, 0, 0);
+    }
+    if (j0 + 31 > pos0 || j0 + 31 >= kv_end) {
+#pragma unroll
+      for (int g = 0; g < kQG; ++g)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int kj = j0 + 8 * (i >> 2) + 4 * half + (i & 3);
+          if (kj > qpos[g] || kj >= kv_end) s[g][i] = -INFINITY;
+        }
+    }
+    float smax[kQG], thr[kQG];
+    bool up[kQG];
+#pragma unroll
+    for (int g = 0; g < kQG; ++g) {
+      float v = s[g][0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) v = fmaxf(v, s[g][i]);
+      const float2 h = halves(v);
+      smax[g] = fmaxf(h.x, h.y);
+      thr[g] = m[g] == -INFINITY ? -INFINITY : kLazyRescale;
+      up[g] = smax[g] > thr[g];
+    }
+    // Lazy rescaling: m is raised -- o and lacc rescaled by 2^(m_old - m_new),
+    // the block's scores shifted, negm reloaded -- only when some column's
+    // block maximum exceeds it by more than kLazyRescale (log2 units), or on
+    // a column's first unmasked key.  Otherwise p = 2^s <= 2^8, well inside
+    // fp32 and bf16.  In exact arithmetic the result does not depend on the
+    // reference; the wave merge below combines each wave's (m, l, o) by its
+    // own reference.  A column whose keys are all masked so far keeps
+    // m = -inf and p = 0.
+    if (__builtin_amdgcn_ballot_w64(up[0] || up[1]) != 0) {
+#pragma unroll
+      for (int g = 0; g < kQG; ++g) {
+        const float cur = m[g] == -INFINITY ? 0.f : m[g];
+        const float mn = up[g] ? fmaxf(m[g], smax[g] + cur) : m[g];
+        const float corr = (up[g] && m[g] != -INFINITY) ? fast_exp2(m[g] - mn) : 1.f;
+        const float d = up[g] ? mn - cur : 0.f;
+        const float nm = mn == -INFINITY ? 0.f : -mn;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          s[g][i] -= d;
+          o[g][i] *= corr;
+          lacc[g][i] *= corr;
+          negm[g][i] = nm;
+        }
+        m[g] = mn;
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < kQG; ++g) {
+      float pf[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) pf[i] = fast_exp2(s[g][i]);
+      uint4 u0, u1;
+      u0.x = pack_bf16x2(pf[0], pf[1]);   u0.y = pack_bf16x2(pf[2], pf[3]);
+      u0.z = pack_bf16x2(pf[4], pf[5]);   u0.w = pack_bf16x2(pf[6], pf[7]);
+      u1.x = pack_bf16x2(pf[8], pf[9]);   u1.y = pack_bf16x2(pf[10], pf[11]);
+      u1.z = pack_bf16x2(pf[12], pf[13]); u1.w = pack_bf16x2(pf[14], pf[15]);
+      pb0[g] = __builtin_bit_cast(bf16x8_t, u0);
+      pb1[g] = __builtin_bit_cast(bf16x8_t, u1);
+    }
+    // V^T as the A operand: lane = dim (col), k-slot e of MFMA b holds key
+    // 16*b + 8*(e/4) + 4*half + (e%4), matching P's register order.  The V
+    // tile is this wave's own: its LDS writes are complete (lgkmcnt) before
+    // its lanes read each other's entries.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    const short4_t a0 = vt_read(0), a1 = vt_read(1), b0 = vt_read(2), b1 = vt_read(3);
+    bf16x8_t va0, va1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      va0[e] = a0[e]; va0[4 + e] = a1[e];
+      va1[e] = b0[e]; va1[4 + e] = b1[e];
+    }
+#pragma unroll
+    for (int g = 0; g < kQG; ++g) {
+      o[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va0, pb0[g], o[g], 0, 0, 0);
+      o[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va1, pb1[g], o[g], 0, 0, 0);
+      lacc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb0[g], lacc[g], 0, 0, 0);
+      lacc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb1[g], lacc[g], 0, 0, 0);
+    }
+    // The next block's V writes come after these reads in program order.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  // This wave's key blocks (wave, wave + kPrefillWaves, ...) stream through
+  // a kPrefillRing-entry register ring: its block i + kPrefillRing - 1 is in
+  // flight while block i is computed, and the page ids of block
+  // i + kPrefillRing with it (ids[i % kPrefillRing]).  Loads past the last
+  // block are clamped to key kv_end - 1 (in bounds) and left unused.
+  const int nblk = (kv_end + 31) / 32;
+  const int nmine = nblk > wave ? (nblk - wave + kPrefillWaves - 1) / kPrefillWaves : 0;
+  auto key0 = [&](int i) { return 32 * (wave + kPrefillWaves * i); };
   constexpr int R = kPrefillRing;
+  KV ring[R];
+  int ids[R];
+  if (a.tile_ints == 12) {
+    // The first R blocks' page ids come with the tile descriptor (entries
+    // 4 + j0 / 16 and the next: pages min(j0, kv_end - 1) / 16 and
+    // min(j0 + 16, kv_end - 1) / 16, as id_of reads them), so their K/V
+    // loads follow the descriptor's round trip directly.
+    static_assert(32 * (kPrefillWaves * (kPrefillRing - 1) + kPrefillWaves - 1) / 16 + 1 < 8, "descriptor pages");
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int k = key0(u) / 16;
+      const int pa = min(max(td[4 + k], 0), a.num_pages - 1);
+      const int pb = min(max(td[5 + k], 0), a.num_pages - 1);
+      ids[u] = col < 16 ? pa : pb;
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < R; ++u) ids[u] = id_of(key0(u));
+  }
+#pragma unroll
+  for (int u = 0; u < R - 1; ++u) load_block(key0(u), ids[u], ring[u]);
+  for (int i0 = 0; i0 < nmine; i0 += R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      ids[u] = id_of(key0(i0 + u + R));
+      load_block(key0(i0 + u + R - 1), ids[(u + R - 1) % R], ring[(u + R - 1) % R]);
+      if (i0 + u < nmine) compute_block(key0(i0 + u), ring[u]);
+    }
+  }
+
+  // Merge the waves' (m, l, o) per query column; a wave without blocks has
+  // m = -inf and contributes nothing.  Wave 0 always holds key 0.
+  __shared__ float pm_all[HPW][kPrefillWaves][kQG][64], pl_all[HPW][kPrefillWaves][kQG][64];
+  __shared__ f32x16_t po_all[HPW][kPrefillWaves - 1][kQG][64];
+#pragma unroll
+  for (int g = 0; g < kQG; ++g) {
+    pm_all[hsub][wave][g][lane] = m[g];
+    pl_all[hsub][wave][g][lane] = lacc[g][0];
+    if (wave > 0) po_all[hsub][wave - 1][g][lane] = o[g];
+  }
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int g = 0; g < kQG; ++g) {
+    float l = lacc[g][0];
+    float M = m[g];
+#pragma unroll
+    for (int w = 1; w < kPrefillWaves; ++w) M = fmaxf(M, pm_all[hsub][w][g][lane]);
+    {
+      const float c0 = fast_exp2(m[g] - M);
+      l *= c0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[g][i] *= c0;
+    }
+#pragma unroll
+    for (int w = 1; w < kPrefillWaves; ++w) {
+      const float c = fast_exp2(pm_all[hsub][w][g][lane] - M);
+      l += pl_all[hsub][w][g][lane] * c;
+      const f32x16_t ow = po_all[hsub][w - 1][g][lane];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[g][i] += ow[i] * c;
+    }
+    // o[g][i]: dim 8*(i/4) + 4*half + (i%4) of query 32 g + col.
+    // Dims 8 b + 4 half .. + 3 are o[g][4 b .. 4 b + 3]: one 8-byte (bf16) or
+    // 16-byte (fp32) store each (ldo % 4 == 0 and a 16-byte aligned out).
+    const int qi = 32 * g + col;
+    if (qi < nvalid) {
+      const float inv = 1.f / l;
+      const int64_t ob = (int64_t)(row0 + qi) * a.ldo + head * kHD + 4 * half;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const float v0 = o[g][4 * b] * inv, v1 = o[g][4 * b + 1] * inv, v2 = o[g][4 * b + 2] * inv,
+                    v3 = o[g][4 * b + 3] * inv;
+        if (a.out_bf16)
+          *(uint2*)((uint16_t*)a.out + ob + 8 * b) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+        else
+          *(float4*)((float*)a.out + ob + 8 * b) = make_float4(v0, v1, v2, v3);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Prefill over long contexts: the same tile and MFMA shapes with NWH = 4 waves
+// per head and K/V through LDS.
+//
+// K/V come into an LDS ring with direct-to-LDS loads in whole cache lines: the
+// two heads of a workgroup are 128 consecutive bytes of a token, and the two
+// waves that work on one key block (one per head) share its ring slot, one
+// loading K and the other V.  The kernel's long contexts are bound by the L2
+// requests (89% of them hit): with a key per lane in the operand layout, or with
+// a 64-byte head slice per wave, each line is asked for twice or more (one
+// layer, 512 rows after 16384 tokens, 64 heads: 198 us in paged_prefill_kernel,
+// 164 with four waves per head there, 149 with 64-byte DMA rows, of which the
+// loads alone took 144 and the arithmetic alone 109; 128 so).
+// ---------------------------------------------------------------------------
+constexpr int kLongWaves = 4;  // waves per head
+constexpr int kLongRing = 3;   // K/V blocks per key-block lane in LDS: one computed, the others in flight
+// The softmax reference lies this far above the largest score seen when it was
+// set, so that a p within the lazy rescale's headroom is below 2.
+constexpr float kLazyLead = kLazyRescale - 1.f;
+
+template <int HPW>
+__global__ __launch_bounds__(HPW * kLongWaves * 64, 2) void paged_prefill_long_kernel(const PrefillArgs a,
+                                                                                     const DecodeArgs merge,
+                                                                                     int merge_rows,
+                                                                                     unsigned prefill_blocks) {
+  if (blockIdx.x >= prefill_blocks) {
+    decode_merge(merge, merge_rows, (int64_t)(blockIdx.x - prefill_blocks) * blockDim.x + threadIdx.x);
+    return;
+  }
+  constexpr int R = kLongRing, NWH = kLongWaves;
   constexpr int RB = 64 * HPW;           // bytes of a key's K (or V) of the workgroup's heads
   constexpr int VOFS = 32 * RB;          // a block: 32 keys of K, then of V
   constexpr int BLOCK = 2 * VOFS;
@@ -861,11 +1217,12 @@ __global__ __launch_bounds__(HPW * NWH * 64, 2) void paged_prefill_kernel(const 
     // i - 1 are done: that slot takes block i + R - 1.
     wait_dma_tile<4, R>(max(min(nmine - 1, i + R - 2) - i, 0));
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (i + R - 1 < nmine) issue_next(i + R - 1, slot == 0 ? (R - 1) * BLOCK : slot - BLOCK);
     if (i >= nmine) continue;
     const int j0 = 32 * (wave + NWH * i);
+    // The next loads are issued under the score MFMAs (a DMA instruction can
+    // hold its wave for tens of cycles).
     uint8_t* const blk = ring + slot;
-    const bf16x8_t k0 = *(const bf16x8_t*)(blk + kofs0), k1 = *(const bf16x8_t*)(blk + kofs1);
+    bf16x8_t k0 = *(const bf16x8_t*)(blk + kofs0), k1 = *(const bf16x8_t*)(blk + kofs1);
     short4_t vt[4];
 #pragma unroll
     for (int mm = 0; mm < 4; ++mm)
@@ -881,6 +1238,8 @@ __global__ __launch_bounds__(HPW * NWH * 64, 2) void paged_prefill_kernel(const 
     f32x16_t s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k0, qb0[1], negm[1], 0, 0, 0);
     s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb1[0], s0, 0, 0, 0);
     s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb1[1], s1, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + R - 1 < nmine) issue_next(i + R - 1, slot == 0 ? (R - 1) * BLOCK : slot - BLOCK);
     // Only blocks reaching past the tile's first query position or past kv_end
     // need the causal mask.
     if (j0 + 31 > pos0 || j0 + 31 >= kv_end) {
@@ -1482,21 +1841,26 @@ int prefill_launch(const cbis_attn_desc* d, int n_tiles, const int* tiles, hipSt
   a.n_heads = d->n_heads;
   a.max_kv = (int)std::min<int64_t>(d->bt_stride * kPS, 1 << 30);
   a.qscale = kLog2e / sqrtf((float)kHD);
-  // Two heads per workgroup, two waves per head; four per head when the grid
-  // gives no CU a second workgroup.
+  // Two heads per workgroup.  Sequences that may be long (the table is as wide as
+  // the longest) take the four-wave kernel where the grid gives no CU a second
+  // two-wave workgroup: its barriers and LDS reads cost more than its loads save
+  // on short ones (64 heads, two waves / four, us a layer: 512 rows after 0, 1024,
+  // 4096, 16384 tokens 9.3 / 11.3, 17.2 / 18.2, 40.9 / 39.2, 198 / 128; 64 rows
+  // after 1024, 16384 13.1 / 15.3, 133 / 118) and it does not fit a CU twice (two
+  // 512-row chunks, 512 workgroups: 14.6 / 24.8).
   const int hpw = d->n_heads % 2 == 0 ? 2 : 1;
   const int64_t pgrid = (int64_t)n_tiles * (d->n_heads / hpw);
-  const int nwh = pgrid <= 256 ? 4 : 2;
-  const int block = hpw * nwh * 64;
+  const bool lng = pgrid <= 256 && d->bt_stride * kPS > 4096;
+  const int block = hpw * (lng ? kLongWaves : kPrefillWaves) * 64;
   const DecodeArgs none = {};
   const int64_t mgrid = merge_rows > 0 ? cdiv((int64_t)merge_rows * m->n_heads * kHD, block) : 0;
   CBIS_REQUIRE(pgrid + mgrid < (1LL << 31), CBIS_ERR_UNSUPPORTED, "%s: grid too large", who);
   const DecodeArgs& mm = merge_rows > 0 ? *m : none;
   const unsigned grid = (unsigned)(pgrid + mgrid);
-  if (hpw == 2 && nwh == 2) paged_prefill_kernel<2, 2><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
-  else if (hpw == 2) paged_prefill_kernel<2, 4><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
-  else if (nwh == 2) paged_prefill_kernel<1, 2><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
-  else paged_prefill_kernel<1, 4><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
+  if (hpw == 2 && lng) paged_prefill_long_kernel<2><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
+  else if (hpw == 2) paged_prefill_kernel<2><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
+  else if (lng) paged_prefill_long_kernel<1><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
+  else paged_prefill_kernel<1><<<grid, block, 0, s>>>(a, mm, merge_rows, (unsigned)pgrid);
   return check_launch(who);
 }
 

@@ -1517,6 +1517,61 @@ def test_prefill_attention_lazy_rescale(cbis, oracle, dev, mode):
     assert err_head < LOWP_TOL * 2
 
 
+@pytest.mark.parametrize("H,qscale", [(2, 1.0), (3, 16.0), (8, 16.0)])
+@pytest.mark.parametrize("tile_pages", [0, 8])
+def test_prefill_attention_long(cbis, oracle, dev, H, qscale, tile_pages):
+    """Prefill tiles under a block table of more than 4096 keys (the four-wave
+    kernel) against the fp64 oracle and the same tiles under a narrow table:
+    one key, last key block of 1, 16, 17, 31 and 32 keys, fewer blocks than
+    waves, ids reloaded after 32 blocks of a wave, several tiles, even and odd
+    head counts, queries that raise the softmax reference after the first
+    block.  NaN past every sequence's end must not reach a row."""
+    import torch
+    seqs = [(0, 1), (0, 16), (16, 1), (0, 31), (3, 61), (100, 64), (95, 33), (1000, 70), (4500, 45)]  # cached, rows
+    D, g = H * 32, rng(40 + H)
+    kv = [a + n for a, n in seqs]
+    npages = [-(-n // 16) for n in kv]
+    P = sum(npages) + 3
+    perm = g.permutation(P).astype(np.int32)
+    wide = np.zeros((len(seqs), max(max(npages), 300)), np.int32)
+    kp, vp = (bf16_dev(g.standard_normal((P, 16, H, 32)).astype(np.float32), dev) for _ in range(2))
+    tiles, pos, row_seq, at, row = [], [], [], 0, 0
+    for s, (cached, n) in enumerate(seqs):
+        wide[s, : npages[s]] = perm[at: at + npages[s]]
+        at += npages[s]
+        if kv[s] % 16:
+            for t in (kp, vp):
+                t[0][int(wide[s, npages[s] - 1]), kv[s] % 16:] = float("nan")
+        for r in range(0, n, 64):
+            m = min(64, n - r)
+            ids = [int(wide[s, min(16 * k, cached + r + m - 1) // 16]) for k in range(8)]
+            tiles.append([row + r, m, s, cached + r] + (ids if tile_pages else []))
+        pos += range(cached, cached + n)
+        row_seq += [s] * n
+        row += n
+    q = (g.standard_normal((row, D)) * qscale).astype(np.float32)
+    # The kernel's Q: scaled by log2(e) / sqrt(32), then rounded to bf16 (at
+    # qscale 16 that rounding alone moves a score by up to 0.1).
+    c = np.float32(1.4426950408889634) / np.sqrt(np.float32(32))
+    qr = bf16_dev(q * c, dev)[1] / c
+    ref = oracle.paged_attention(qr, kp[1], vp[1], wide[row_seq], np.array(pos, np.int32), H, 32, 16)
+    Q, T = to_dev(q, dev), to_dev(np.array(tiles, np.int32), dev)
+    outs = []
+    for width in (wide.shape[1], 256):
+        keep = [i for i, k in enumerate(kv) if k <= width * 16]
+        sel = [i for i, t in enumerate(tiles) if t[2] in keep]
+        BT, TS = to_dev(np.ascontiguousarray(wide[:, :width]), dev), T[sel].contiguous()
+        out = torch.full((row, D), 7.0, dtype=torch.float32, device=dev)
+        d = _attn_desc(cbis, 0, H, Q, kp[0], vp[0], P, BT, width, None, out, cbis.BF16)
+        d.tile_pages = tile_pages
+        cbis.check(cbis.kernels().cbis_paged_prefill_attention(ctypes.byref(d), len(sel), ptr(TS), stream()))
+        sync()
+        outs.append(out.cpu().numpy())
+    assert row_rel_err(outs[0].reshape(row, -1), ref.reshape(row, -1)) < LOWP_TOL
+    same = np.isin(row_seq, keep)
+    assert same.sum() > 200 and row_rel_err(outs[0][same], outs[1][same]) < LOWP_TOL
+
+
 @pytest.mark.parametrize("H", [1, 8, 12])
 @pytest.mark.parametrize("qdt,odt", [("f32", "f32"), ("bf16", "bf16")])
 def test_chunk_attention_f32(cbis, oracle, dev, H, qdt, odt):
