@@ -1312,14 +1312,18 @@ __global__ __launch_bounds__(512) void gemm_bf16_ws_kernel(const GemmArgs g) {
   }
 }
 
-template <typename WT, int BM, int BN, int STAGES, int REGS = 0, int WM = 2>
+// GREEDY: the tiling also has its greedy-mode instantiation (choose_bf16's).
+template <typename WT, int BM, int BN, int STAGES, int REGS = 0, int WM = 2, bool GREEDY = true>
 int launch_ws(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = cdiv(g.M, BM) * cdiv(g.N, BN);
-  if (g.amax)
-    gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, true><<<dim3((unsigned)tiles, 1, 1), 512, 0, s>>>(g);
-  else
-    gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, false>
-        <<<dim3((unsigned)tiles, 1, g.ksplit), 512, 0, s>>>(with_vec(g));
+  if constexpr (GREEDY) {
+    if (g.amax) {
+      gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, true><<<dim3((unsigned)tiles, 1, 1), 512, 0, s>>>(g);
+      return check_launch("cbis_gemm(bf16 ws)");
+    }
+  }
+  gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, false>
+      <<<dim3((unsigned)tiles, 1, g.ksplit), 512, 0, s>>>(with_vec(g));
   return check_launch("cbis_gemm(bf16 ws)");
 }
 
@@ -1697,12 +1701,8 @@ int launch_skinny(const GemmArgs& g, hipStream_t s) {
 
 constexpr int kSkinnyMaxM = 64;
 
-// Tile of the bf16 direct-to-LDS path and its split-K plan.  The tile is
-// 128 x 128 on 8 waves (2 x 4, each 64 x 32) with a 2-stage 64 KiB ring, so
-// two workgroups share a CU.  When the output tiles cannot occupy the 256 CUs
-// and K has at least 64 tiles, K is split so about 2 workgroups per CU run;
-// each split keeps at least 16 K tiles.  (Measured: at K = 2048 the partial
-// round trip costs more than the occupancy gains.)
+// The larger tile of gemm_bf16_dma_kernel: 128 x 128 on 8 waves (2 x 4, each
+// 64 x 32) with a 2-stage 64 KiB ring, so two workgroups share a CU.
 constexpr int kDmaBM = 128, kDmaBN = 128;
 constexpr int kCUs = 256;
 
@@ -1713,11 +1713,11 @@ struct SplitPlan {
 
 // Kernel for a bf16 or fp8 W on the direct-to-LDS paths, from the
 // tile counts (measured on config 4's shapes at M = 1216, TFLOP/s):
-//   < kCUs / 2 tiles of 128 x 128, or K < 512: gemm_bf16_dma_kernel, 64 x 64
-//     tiles or 128 x 128 with split-K (plan_dma_split); with under 8 K tiles
-//     the wave-specialised kernel's ring fill and parked epilogue cost more
-//     than they save (config 2, M = 4096, K = 256: 9.5 / 14.1 us against
-//     10.8 / 19.1);
+//   < kCUs / 2 tiles of 128 x 128, or K < 512: gemm_bf16_dma_kernel (here only
+//     with K < kRoundMinK: plan_round comes first); with under 8 K tiles the
+//     wave-specialised kernel's ring fill and parked epilogue cost more than
+//     they save (config 2, M = 4096, K = 256: 9.5 / 14.1 us against 10.8 /
+//     19.1);
 //   < kCUs tiles and K of 96 tiles of 64 or more: 160 x 256 tiles with
 //     split-K into up to 4 parts, about one workgroup per CU.  With weights
 //     cold in HBM, as in the step, this beats whole-K tilings (fc2 at
@@ -1760,26 +1760,92 @@ Bf16Path choose_bf16(int M, int N, int K) {
   return Bf16Path::kWs128R;
 }
 
+// Wave-specialised tilings for grids that one round of workgroups, at most one
+// per CU, can cover (decode batches of 33 rows on, short prompt chunks).  Such
+// calls stream their weights once and are bound by the latency of a K tile --
+// its barrier, LDS reads and MFMA chain -- times the K tiles of a workgroup, so
+// the smallest tile that still fits the round wins, and K is split as far as
+// the round allows: the model is K tiles per workgroup times the tile's time,
+// plus the partials' traffic.  Times per K tile fitted on M = 48..512 of the
+// mid-size layer's four shapes (weights cold; qkv / out / fc1 / fc2 in us, LayerNorms
+// included, before and after: M = 64 bf16 17 / 12.6 / 25 / 28 -> 10 / 9.7 / 12 / 16,
+// M = 192 bf16 16 / 20 / 21 / 37 -> 13 / 11 / 16 / 22, fp8 16 / 18 / 17 / 27 ->
+// 13 / 11 / 14 / 18, M = 512 bf16 20 / 19 / 30 / 41 -> 20 / 16 / 25 / 34).
+enum class RoundTile { kNone, k64x64, k64x128, k128x64, k96x128, k128x128 };
+struct RoundPlan {
+  RoundTile tile = RoundTile::kNone;
+  SplitPlan split;
+};
+
+constexpr int kRoundMinK = 1024;  // below, the ring fill costs more than the kernel saves
+constexpr int kSplitMinK = 4096;  // a plain call, whose reduce is a launch of its own, splits K from here on
+
+// max_split: the most K parts (1, or 4: the most the reduce kernels take).
+RoundPlan plan_round(int M, int N, int K, int w_dtype, int max_split) {
+  RoundPlan best;
+  best.split.k_per = K;
+  if (K < kRoundMinK || K % 64) return best;
+  struct Cand {
+    RoundTile tile;
+    int bm, bn;
+    double bf16_us, fp8_us;  // per K tile of 64
+  };
+  static constexpr Cand kCands[] = {{RoundTile::k64x64, 64, 64, 0.23, 0.22},
+                                    {RoundTile::k128x64, 128, 64, 0.33, 0.30},
+                                    {RoundTile::k64x128, 64, 128, 0.34, 0.28},
+                                    {RoundTile::k96x128, 96, 128, 0.44, 0.37},
+                                    {RoundTile::k128x128, 128, 128, 0.53, 0.47}};
+  const int kt = K / 64;
+  const double part_us = 8e-6 * M * N / 6.0;  // write and read of one part at 6 TB/s
+  double t_best = 1e30;
+  for (const Cand& c : kCands) {
+    const int64_t tiles = cdiv(M, c.bm) * cdiv(N, c.bn);
+    for (int ks = 1; ks <= max_split && tiles * ks <= kCUs; ++ks) {
+      const int per = (kt + ks - 1) / ks;
+      if (ks > 1 && (per < 8 || (kt + per - 1) / per != ks)) continue;
+      const double t = per * (w_dtype == CBIS_BF16 ? c.bf16_us : c.fp8_us) + ks * part_us;
+      if (t < t_best) {
+        t_best = t;
+        best.tile = c.tile;
+        best.split.ksplit = ks;
+        best.split.k_per = per * 64;
+      }
+    }
+  }
+  return best;
+}
+
+// choose_bf16's own split-K (grids that plan_round does not take).
 SplitPlan plan_dma_split(int M, int N, int K) {
   SplitPlan p;
   p.k_per = K;
-  const int64_t tiles = cdiv(M, kDmaBM) * cdiv(N, kDmaBN);
-  const int kt = K / 64;
-  const Bf16Path path = choose_bf16(M, N, K);
-  if (path == Bf16Path::kWs160Split) {
-    const int ks = ws160_splits(M, N, K);
-    const int per = (kt + ks - 1) / ks;
-    p.ksplit = (kt + per - 1) / per;
-    p.k_per = per * 64;
-    return p;
-  }
-  if (path != Bf16Path::kSmall || tiles >= kCUs || kt < 64) return p;
-  int ks = (int)std::max<int64_t>(2, std::min<int64_t>(4, (2 * kCUs) / tiles));
-  ks = std::min(ks, kt / 16);
-  if (ks <= 1) return p;
-  const int per = (kt + ks - 1) / ks;
+  if (choose_bf16(M, N, K) != Bf16Path::kWs160Split) return p;
+  const int kt = K / 64, ks = ws160_splits(M, N, K), per = (kt + ks - 1) / ks;
   p.ksplit = (kt + per - 1) / per;
   p.k_per = per * 64;
+  return p;
+}
+
+// The tiling and split of a call on the direct-to-LDS paths.  fused_reduce: the
+// partials are summed by the LayerNorm kernel that follows, so a split costs no
+// launch.
+struct DmaPlan {
+  RoundTile round = RoundTile::kNone;  // kNone: choose_bf16's path
+  SplitPlan split;
+};
+
+DmaPlan plan_dma(int M, int N, int K, int w_dtype, bool fused_reduce, bool may_split) {
+  DmaPlan p;
+  const bool deep_wide = choose_bf16(M, N, K) == Bf16Path::kWs160Split;
+  if (!deep_wide) {
+    const RoundPlan r =
+        plan_round(M, N, K, w_dtype, may_split && (fused_reduce || K >= kSplitMinK) ? 4 : 1);
+    p.round = r.tile;
+    p.split = r.split;
+    if (r.tile != RoundTile::kNone) return p;
+  }
+  p.split.k_per = K;
+  if (may_split) p.split = plan_dma_split(M, N, K);
   return p;
 }
 
@@ -1870,10 +1936,19 @@ int dispatch(const GemmArgs& g, hipStream_t s) {
   }
 }
 
-// Launches the direct-to-LDS kernel that choose_bf16 picks, on g's split.
+// Launches the direct-to-LDS kernel of the plan (greedy mode: choose_bf16's) on
+// g's split.
 template <typename WT>
-int dispatch_dma(const GemmArgs& g, hipStream_t s) {
+int dispatch_dma(const GemmArgs& g, RoundTile round, hipStream_t s) {
   const bool split = g.ksplit > 1;
+  switch (round) {
+    case RoundTile::k64x64: return launch_ws<WT, 64, 64, 4, 0, 2, false>(g, s);
+    case RoundTile::k64x128: return launch_ws<WT, 64, 128, 4, 0, 1, false>(g, s);
+    case RoundTile::k128x64: return launch_ws<WT, 128, 64, 4, 0, 2, false>(g, s);
+    case RoundTile::k96x128: return launch_ws<WT, 96, 128, 4, 0, 1, false>(g, s);
+    case RoundTile::k128x128: return launch_ws<WT, 128, 128, 4, 0, 2, false>(g, s);
+    case RoundTile::kNone: break;
+  }
   switch (choose_bf16(g.M, g.N, g.K)) {
     case Bf16Path::kWs256: return launch_ws<WT, 128, 256, 3>(g, s);
     case Bf16Path::kWs160: return launch_ws<WT, 160, 256, 3, 0, 1>(g, s);
@@ -1898,15 +1973,28 @@ int dispatch_dma(const GemmArgs& g, hipStream_t s) {
   return launch_dma<WT, kDmaBM, kDmaBN, 2, 4, 2>(g, s);
 }
 
+// Whether d's GEMM can run on the skinny (decode-sized) kernel.
+bool skinny_path(const cbis_gemm_desc* d) {
+  const int we = d->w_dtype == CBIS_F32 ? 4 : (d->w_dtype == CBIS_BF16 ? 2 : 1);
+  const bool w_al = ((uintptr_t)d->W & 15u) == 0 && (d->ldw * we) % 16 == 0;
+  return d->M <= kSkinnyMaxM && w_al && d->K % (d->w_dtype == CBIS_FP8E4M3 ? 64 : 32) == 0;
+}
+
+// Whether a greedy call does: up to 32 rows, and of 33..64 rows those that have
+// no wave-specialised tiling (lm_head 32000 x 2048, bf16: 40 rows 67 us skinny,
+// 80 rows 26 on the tiles).
+bool greedy_skinny(const cbis_gemm_desc* d) {
+  return skinny_path(d) && (d->M <= 32 || !dma_eligible(d) || d->K < kRoundMinK ||
+                            choose_bf16(d->M, d->N, d->K) == Bf16Path::kSmall);
+}
+
 // Column-tile width of the greedy-mode partials for d's GEMM path: the
 // kernels that reduce in their epilogue are the skinny one (16 columns per
 // workgroup) and the wave-specialised ones (their BN); 0 for the others
 // (fp32 weights at M > 64, small grids, unaligned W), whose logits
 // cbis_gemm_argmax stores and reduces instead.  Follows gemm_run's choice.
 int argmax_tile_cols(const cbis_gemm_desc* d) {
-  const int we = d->w_dtype == CBIS_F32 ? 4 : (d->w_dtype == CBIS_BF16 ? 2 : 1);
-  const bool w_al = ((uintptr_t)d->W & 15u) == 0 && (d->ldw * we) % 16 == 0;
-  if (d->M <= kSkinnyMaxM && w_al && d->K % (d->w_dtype == CBIS_FP8E4M3 ? 64 : 32) == 0) return 16;
+  if (greedy_skinny(d)) return 16;
   if (!dma_eligible(d)) return 0;
   switch (choose_bf16(d->M, d->N, d->K)) {
     case Bf16Path::kWs256:
@@ -1934,24 +2022,28 @@ struct LnPrologue {
   float eps;
 };
 
-// Whether d's GEMM runs on the skinny (decode-sized) kernel.
-bool skinny_path(const cbis_gemm_desc* d) {
-  const int we = d->w_dtype == CBIS_F32 ? 4 : (d->w_dtype == CBIS_BF16 ? 2 : 1);
-  const bool w_al = ((uintptr_t)d->W & 15u) == 0 && (d->ldw * we) % 16 == 0;
-  return d->M <= kSkinnyMaxM && w_al && d->K % (d->w_dtype == CBIS_FP8E4M3 ? 64 : 32) == 0;
-}
-
 // Whether a plain call (no greedy epilogue, LayerNorm prologue or fused
-// split-K reduce, which are the skinny kernel's own) of decode-sized M runs
-// on the skinny kernel: always up to 32 rows; bf16 x bf16 calls of 33..64
-// rows take the direct-to-LDS tiles instead, whose workgroups read X once
-// per tile where the skinny kernel reads all of it once per 16 columns
-// (config 2 at M = 64, qkv / out / MLP up / MLP down: 7.0 / 7.0 / 7.6 / 10.4
-// us skinny, 4.2 / 4.2 / 4.7 / 7.0 tiled).  fp32 weights keep the skinny
-// kernel (M = 64 qkv 8.3 us against 9.1 on the fp32 tiles), fp8 weights too.
+// split-K reduce) of decode-sized M runs on the skinny kernel: always up to 32
+// rows; of 33..64 rows those with bf16 or fp8 weights take the direct-to-LDS
+// tiles instead, whose workgroups read X once per tile where the skinny kernel
+// reads all of it once per 16 columns (d 256, bf16, M = 64, qkv / out / MLP up / MLP
+// down: 7.0 / 7.0 / 7.6 / 10.4 us skinny, 4.2 / 4.2 / 4.7 / 7.0 tiled; d 2048, fp8, M
+// = 48, qkv / MLP up 18.9 / 19.5 skinny, 10.2 / 10.7 tiled).  fp32 weights keep the
+// skinny kernel (M = 64 qkv 8.3 us against 9.1 on the fp32 tiles), and so do
+// fp8 ones with short K, which plan_round leaves to the older tiles, or with a K
+// so deep that the tiles would need its split.
 bool plain_skinny(const cbis_gemm_desc* d) {
-  return skinny_path(d) && (d->M <= 32 || d->w_dtype != CBIS_BF16 || !dma_eligible(d));
+  if (!skinny_path(d)) return false;
+  if (d->M <= 32 || !dma_eligible(d)) return true;
+  return d->w_dtype != CBIS_BF16 && (d->K < kRoundMinK || d->K >= kSplitMinK);
 }
+// The same for a call whose LayerNorm kernel sums the partials
+// (cbis_gemm_layernorm): the tiles split K there at any depth.
+bool fused_skinny(const cbis_gemm_desc* d) {
+  return skinny_path(d) && (d->M <= 32 || !dma_eligible(d) || d->K < kRoundMinK);
+}
+// Whether a plain call on the direct-to-LDS paths may split K.
+bool plain_may_split(const cbis_gemm_desc* d) { return d->M > kSkinnyMaxM || d->w_dtype == CBIS_BF16; }
 
 // Whether cbis_layernorm_gemm(_argmax) forms d's LayerNorm inside the GEMM.
 bool ln_prologue_ok(const cbis_gemm_desc* d, const float* x, int64_t ldx, const float* gamma, const float* beta) {
@@ -2023,7 +2115,7 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
 
   // Decode-sized M: weight streaming (K a multiple of 32 for bf16 and fp32,
   // of 64 for fp8; W rows 16-byte aligned).
-  if (amax || ln || fused_reduce ? skinny_path(d) : plain_skinny(d)) {
+  if (ln ? skinny_path(d) : amax ? greedy_skinny(d) : fused_reduce ? fused_skinny(d) : plain_skinny(d)) {
     if (fused_reduce && !amax && !ln) {
       const SplitPlan p = plan_skinny_split(d->M, d->N, d->K, d->w_dtype);
       const size_t need = (size_t)p.ksplit * d->M * d->N * sizeof(float);
@@ -2049,14 +2141,21 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
   }
   // The direct-to-LDS path needs 16-byte aligned rows of both operands.
   if (dma_eligible(d)) {
-    const SplitPlan p = plan_dma_split(d->M, d->N, d->K);
-    const size_t need = (size_t)p.ksplit * d->M * d->N * sizeof(float);
-    if (!amax && p.ksplit > 1 && d->workspace && d->workspace_bytes >= need) {
-      g.ksplit = p.ksplit;
-      g.k_per = p.k_per;
-      g.partial = (float*)d->workspace;
+    DmaPlan p;
+    if (!amax) {
+      p = plan_dma(d->M, d->N, d->K, d->w_dtype, fused_reduce, plain_may_split(d) || fused_reduce);
+      if (p.split.ksplit > 1) {
+        const size_t need = (size_t)p.split.ksplit * d->M * d->N * sizeof(float);
+        if (d->workspace && d->workspace_bytes >= need) {
+          g.ksplit = p.split.ksplit;
+          g.k_per = p.split.k_per;
+          g.partial = (float*)d->workspace;
+        } else {
+          p = plan_dma(d->M, d->N, d->K, d->w_dtype, fused_reduce, false);
+        }
+      }
     }
-    return d->w_dtype == CBIS_BF16 ? dispatch_dma<uint16_t>(g, s) : dispatch_dma<uint8_t>(g, s);
+    return d->w_dtype == CBIS_BF16 ? dispatch_dma<uint16_t>(g, p.round, s) : dispatch_dma<uint8_t>(g, p.round, s);
   }
   return d->w_dtype == CBIS_BF16 ? dispatch<uint16_t, uint16_t>(g, s) : dispatch<uint16_t, uint8_t>(g, s);
 }
@@ -2219,14 +2318,12 @@ int cbis_layernorm_gemm_argmax(const cbis_gemm_desc* d, const float* x, int64_t 
 size_t cbis_gemm_layernorm_workspace_size(const cbis_gemm_desc* d) {
   if (!d || d->M <= 0 || d->N <= 0 || d->K <= 0) return 0;
   // Skinny calls split only here, where the LayerNorm kernel folds the
-  // partials in (plan_skinny_split).
-  const int we = d->w_dtype == CBIS_F32 ? 4 : (d->w_dtype == CBIS_BF16 ? 2 : 1);
-  if (d->M <= kSkinnyMaxM && ((uintptr_t)d->W & 15u) == 0 && (d->ldw * we) % 16 == 0 &&
-      d->K % (d->w_dtype == CBIS_FP8E4M3 ? 64 : 32) == 0) {
-    const SplitPlan p = plan_skinny_split(d->M, d->N, d->K, d->w_dtype);
-    return p.ksplit > 1 ? (size_t)p.ksplit * d->M * d->N * sizeof(float) : 0;
-  }
-  return cbis_gemm_workspace_size(d);
+  // partials in (plan_skinny_split); so do shallow-K calls on the tiles.
+  SplitPlan p;
+  if (fused_skinny(d)) p = plan_skinny_split(d->M, d->N, d->K, d->w_dtype);
+  else if (dma_eligible(d) && d->K % 64 == 0) p = plan_dma(d->M, d->N, d->K, d->w_dtype, true, true).split;
+  else return cbis_gemm_workspace_size(d);
+  return p.ksplit > 1 ? (size_t)p.ksplit * d->M * d->N * sizeof(float) : 0;
 }
 
 size_t cbis_gemm_workspace_size(const cbis_gemm_desc* d) {
@@ -2241,7 +2338,7 @@ size_t cbis_gemm_workspace_size(const cbis_gemm_desc* d) {
     return p.ksplit > 1 ? (size_t)p.ksplit * d->M * d->N * sizeof(float) : 0;
   }
   if (!dma_eligible(d) || d->K % 64) return 0;
-  const SplitPlan p = plan_dma_split(d->M, d->N, d->K);
+  const SplitPlan p = plan_dma(d->M, d->N, d->K, d->w_dtype, false, plain_may_split(d)).split;
   return p.ksplit > 1 ? (size_t)p.ksplit * d->M * d->N * sizeof(float) : 0;
 }
 

@@ -169,7 +169,7 @@ int cbis_gemm_layernorm(const cbis_gemm_desc* d, const float* ln_gamma, const fl
  * the reference's scan starts from the row's first value, so a NaN there makes
  * the token 0 (its margin is then +inf, or NaN when another logit is +inf).
  * The kernels that reduce in their epilogue
- * (M <= 64, and bf16 or fp8 weights on the wave-specialised tilings) never store Y;
+ * (the skinny one, and bf16 or fp8 weights on the wave-specialised tilings) never store Y;
  * the others store the logits in d->Y (when it is an fp32 [M, N] buffer) or
  * the workspace and reduce them.  The epilogue must be scale and bias only
  * (no GELU, residual or K/V scatter).  workspace: 16-byte aligned, at least

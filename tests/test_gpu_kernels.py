@@ -555,10 +555,73 @@ def test_gemm_fp8_tiles(cbis, oracle, dev, M, N, K, gelu, res):
     assert np.all(np.abs(Y.cpu().numpy()[rows] - ref) <= tol)
 
 
-@pytest.mark.parametrize("M,N,K", [(1216, 8000, 512), (300, 6007, 512), (65, 32000, 2048)])
-def test_gemm_argmax_fp8_tiles(cbis, oracle, dev, M, N, K):
-    """The greedy epilogue of the wave-specialised tiles with fp8 weights."""
-    test_gemm_argmax_matches_logits(cbis, oracle, dev, M, N, K, "fp8")
+@pytest.mark.parametrize("M,N,K,wdt", [(1216, 8000, 512, "fp8"), (300, 6007, 512, "fp8"), (65, 32000, 2048, "fp8"),
+                                       (33, 17000, 1024, "fp8"), (64, 17000, 1024, "bf16")])
+def test_gemm_argmax_tiles(cbis, oracle, dev, M, N, K, wdt):
+    """The greedy epilogue of the wave-specialised tiles with fp8 weights, and
+    of 33..64 rows."""
+    test_gemm_argmax_matches_logits(cbis, oracle, dev, M, N, K, wdt)
+
+
+@pytest.mark.parametrize("wdt", ["bf16", "fp8"])
+@pytest.mark.parametrize("M,N,K,ln", [
+    (33, 252, 1024, False),    # 64 x 64, one row tile
+    (65, 2048, 2048, True),    # 64 x 64, split under the LayerNorm
+    (130, 6148, 1088, False),  # 128 x 64 (bf16) or 64 x 128 (fp8), ragged both ways, 17 K tiles
+    (300, 2052, 4160, True),   # the same, 65 K tiles in uneven parts
+    (384, 6144, 1024, False),  # 96 x 128
+    (384, 2048, 8192, True),   # 96 x 128, split
+    (500, 8192, 1024, False),  # 128 x 128, 256 tiles: the last that fits one round
+    (512, 2048, 8192, False),  # 128 x 128, split, reduce of its own
+    (514, 8192, 1024, False),  # past it
+])
+def test_gemm_one_round_tiles(cbis, oracle, dev, wdt, M, N, K, ln):
+    """Grids of up to one workgroup per CU (plan_round's tiles and splits):
+    x + bias + residual on sampled rows against the product in 64 bits, each of
+    the K + 7 fp32 operations of an output at most 2^-23 of the sum of
+    magnitudes off; with ln, the normalised rows against a LayerNorm of the x
+    written (one bf16 rounding and fp32 statistics)."""
+    import torch
+    X, x = bf16_dev(oracle.normal(91, 1, M * K).reshape(M, K), dev)
+    wf = oracle.normal(91, 2, N * K, 0.02).reshape(N, K)
+    S = None
+    if wdt == "bf16":
+        W, w = bf16_dev(wf, dev)
+        w = w.astype(np.float64)
+    else:
+        codes, sc = oracle.quantize_e4m3_rows(wf)
+        W, S = to_dev(codes, dev), to_dev(sc, dev)
+        w = oracle.e4m3_table()[codes].astype(np.float64) * sc.astype(np.float64)[:, None]
+    b, r = oracle.normal(91, 3, N, 0.02), oracle.normal(91, 4, M * N).reshape(M, N)
+    B, R = to_dev(b, dev), to_dev(r, dev)
+    Y = torch.empty((M, N), dtype=torch.float32, device=dev)
+    d = cbis.GemmDesc()
+    d.M, d.N, d.K = M, N, K
+    d.x_dtype, d.X, d.ldx = cbis.BF16, ptr(X), K
+    d.w_dtype, d.W, d.ldw, d.w_scale = (cbis.BF16 if wdt == "bf16" else cbis.FP8E4M3), ptr(W), K, ptr(S)
+    d.bias, d.residual, d.ldr = ptr(B), ptr(R), N
+    d.y_dtype, d.Y, d.ldy = cbis.F32, ptr(Y), N
+    K_ = cbis.kernels()
+    need = (K_.cbis_gemm_layernorm_workspace_size if ln else K_.cbis_gemm_workspace_size)(ctypes.byref(d))
+    ws = torch.full((need // 4 + 4,), float("nan"), dtype=torch.float32, device=dev)
+    d.workspace, d.workspace_bytes = ptr(ws), need
+    if ln:
+        assert need > 0
+        gam, bet = 1.0 + oracle.normal(91, 5, N, 0.1), oracle.normal(91, 6, N, 0.1)
+        G, Be = to_dev(gam, dev), to_dev(bet, dev)
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+        cbis.check(K_.cbis_gemm_layernorm(ctypes.byref(d), ptr(G), ptr(Be), 1e-5, cbis.BF16, ptr(out), N, stream()))
+    else:
+        cbis.check(K_.cbis_gemm(ctypes.byref(d), stream()))
+    sync()
+    assert torch.isnan(ws[need // 4:]).all()
+    rows = np.unique(np.concatenate([_sample_rows(M, 40, N + K), [0, M - 1]]))
+    xr, got = x[rows].astype(np.float64), Y.cpu().numpy()
+    mag = np.abs(xr) @ np.abs(w).T + np.abs(b) + np.abs(r[rows])
+    assert np.all(np.abs(got[rows] - (xr @ w.T + b + r[rows])) <= (K + 7) * 2.0 ** -23 * mag)
+    if ln:
+        lref = oracle.layernorm(got, gam, bet)
+        assert (np.abs(out.float().cpu().numpy() - lref) / (1.0 + np.abs(lref))).max() < 2 ** -7
 
 
 def test_gemm_fp8_decode_every_code(cbis, oracle, dev):
