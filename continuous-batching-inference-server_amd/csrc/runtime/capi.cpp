@@ -218,8 +218,7 @@ int cbis_runner_forward_step(cbis_runner* r, int n, const int* token_ids, const 
   return guard([&] {
     if (n < 0) throw std::invalid_argument("forward_step: n < 0");
     std::vector<int> t(token_ids, token_ids + n), p(positions, positions + n), s(seq_ids, seq_ids + n);
-    const std::vector<float> lg = r->impl->forward_step(t, p, s);
-    if (!lg.empty()) std::memcpy(logits_out, lg.data(), lg.size() * 4);
+    r->impl->forward_step_into(t, p, s, logits_out);
     return 0;
   });
 }

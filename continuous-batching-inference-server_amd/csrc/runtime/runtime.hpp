@@ -160,6 +160,9 @@ class TransformerRunner {
   // Returns row-major [rows, vocab] logits (the reference's contract).
   std::vector<float> forward_step(const std::vector<int>& token_ids, const std::vector<int>& positions,
                                   const std::vector<int>& seq_ids);
+  // The same into a caller's [rows, vocab] buffer.
+  void forward_step_into(const std::vector<int>& token_ids, const std::vector<int>& positions,
+                         const std::vector<int>& seq_ids, float* logits);
   // Same step; returns the greedy next token of every row.  lm_head runs
   // fused with the row argmax (cbis_gemm_argmax): the logits are not stored
   // where its kernel reduces them in the epilogue.  last_margins() then holds
@@ -250,6 +253,8 @@ class TransformerRunner {
   void* d_attn_ = nullptr;
   void* d_h_ = nullptr;
   float* d_logits_ = nullptr;
+  float *h_logits_ = nullptr, *hd_logits_ = nullptr;  // pinned host memory for small steps' logits, and its device address
+  size_t h_logits_floats_ = 0;
   void* d_amax_ws_ = nullptr;  // cbis_gemm_argmax partials
   size_t amax_ws_bytes_ = 0;
   std::vector<float> margins_;

@@ -31,6 +31,11 @@ constexpr int kMinPrefillRun = 8;   // runs shorter than this use the decode ker
 constexpr int kTileRows = CBIS_PREFILL_TILE_ROWS;  // query rows per prefill tile
 constexpr int kTileInts = 12;  // a prefill tile's descriptor with its first 8 page ids (tile_pages = 8)
 constexpr size_t kMaxGraphs = 64;
+// Logits of up to this many bytes are stored into pinned host memory by the
+// step's last launch and copied to the caller from there.  With a copy command
+// into pageable memory after the step, a zeroed vector and a copy out of it, the
+// whole step took 162 us for 8 x 512 logits (147 so) and 568 for 512 x 1000 (503).
+constexpr size_t kStagedLogits = (size_t)4 << 20;
 size_t align_ints(size_t n) { return (n + 3) & ~(size_t)3; }
 }  // namespace
 
@@ -67,6 +72,10 @@ TransformerRunner::TransformerRunner(const ModelWeights& weights, PagedKVCache& 
   hip_check(hipMalloc(&d_attn_, R * D * ae), "hipMalloc attn");
   hip_check(hipMalloc(&d_h_, R * F * ae), "hipMalloc h");
   hip_check(hipMalloc((void**)&d_logits_, R * V * 4), "hipMalloc logits");
+  h_logits_floats_ = std::min(R * V, kStagedLogits / 4);
+  hip_check(hipHostMalloc((void**)&h_logits_, h_logits_floats_ * 4, hipHostMallocMapped | hipHostMallocCoherent),
+            "hipHostMalloc logits");
+  hip_check(hipHostGetDevicePointer((void**)&hd_logits_, h_logits_, 0), "hipHostGetDevicePointer logits");
   // Split-KV partials: the automatic split keeps rows * splits <= 2048 + rows.
   ws_bytes_ = (2048 + R) * (size_t)cfg_.n_heads * (cfg_.head_dim + 4) * 4;
   hip_check(hipMalloc(&d_ws_, ws_bytes_), "hipMalloc attention workspace");
@@ -107,6 +116,7 @@ TransformerRunner::~TransformerRunner() {
   }
   (void)hipFree(d_x_); (void)hipFree(d_xn_); (void)hipFree(d_q_); (void)hipFree(d_attn_);
   (void)hipFree(d_h_); (void)hipFree(d_logits_);
+  if (h_logits_) (void)hipHostFree(h_logits_);
   (void)hipFree(d_ws_);
   if (d_amax_ws_) (void)hipFree(d_amax_ws_);
   if (d_gemm_ws_) (void)hipFree(d_gemm_ws_);
@@ -436,6 +446,10 @@ void TransformerRunner::enqueue_forward(int b, bool greedy, bool from_prev) {
     cbis_check(cbis_gemm_argmax(&g, d_next, margins, d_amax_ws_, amax_ws_bytes_, s), "lm_head gemm + argmax");
   else
     cbis_check(cbis_gemm(&g, s), "lm_head gemm");
+  // Logits of up to kStagedLogits bytes reach the host without a copy command.
+  const size_t n = (size_t)M * V;
+  if (!greedy && n <= h_logits_floats_)
+    cbis_check(cbis_convert_f32(hd_logits_, CBIS_F32, d_logits_, (int64_t)n, s), "logits to host memory");
 }
 
 void TransformerRunner::run_step(int b, bool greedy, bool from_prev) {
@@ -482,23 +496,31 @@ void TransformerRunner::timed_step(int b, bool greedy, bool from_prev) {
 
 std::vector<float> TransformerRunner::forward_step(const std::vector<int>& token_ids, const std::vector<int>& positions,
                                                    const std::vector<int>& seq_ids) {
+  std::vector<float> logits(token_ids.size() * (size_t)cfg_.vocab);
+  forward_step_into(token_ids, positions, seq_ids, logits.data());
+  return logits;
+}
+
+void TransformerRunner::forward_step_into(const std::vector<int>& token_ids, const std::vector<int>& positions,
+                                          const std::vector<int>& seq_ids, float* logits) {
   margins_.clear();
   const int M = (int)token_ids.size();
-  if (M == 0) return {};
+  if (M == 0) return;
   if ((int)positions.size() != M || (int)seq_ids.size() != M)
     throw std::invalid_argument("forward_step: token_ids/positions/seq_ids sizes differ");
   const int b = next_buf_;
   if (bufs_[b].pending) throw std::logic_error("forward_step: a queued greedy step has not been waited for");
   prepare(b, token_ids.data(), positions.data(), seq_ids.data(), nullptr, M);
   timed_step(b, false, false);
-  std::vector<float> logits((size_t)M * cfg_.vocab);
-  hip_check(hipMemcpyAsync(logits.data(), d_logits_, logits.size() * 4, hipMemcpyDeviceToHost, stream_), "D2H logits");
+  const size_t n = (size_t)M * cfg_.vocab;
+  const bool staged = n <= h_logits_floats_;  // stored in host memory by the step itself
+  if (!staged) hip_check(hipMemcpyAsync(logits, d_logits_, n * 4, hipMemcpyDeviceToHost, stream_), "D2H logits");
   hip_check(hipStreamSynchronize(stream_), "forward_step sync");
   hip_check(hipEventElapsedTime(&last_device_ms_, bufs_[b].ev_start, bufs_[b].ev_stop), "hipEventElapsedTime");
+  if (staged) std::memcpy(logits, h_logits_, n * 4);
   bufs_[b].ticket = -1;
   next_buf_ ^= 1;
   prev_greedy_rows_ = -1;  // no greedy tokens for the next step to read
-  return logits;
 }
 
 int64_t TransformerRunner::enqueue_greedy(const std::vector<int>& token_ids, const std::vector<int>& positions,
