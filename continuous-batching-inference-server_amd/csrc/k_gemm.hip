@@ -639,9 +639,9 @@ __global__ __launch_bounds__(256) void splitk_layernorm_kernel(const GemmArgs g,
 // vector-memory instruction is issued inside the main loop, so the vmcnt
 // immediates count exactly the DMA loads of the younger tiles.
 // ---------------------------------------------------------------------------
-// One stage of the ring: BM rows of X (128 bytes of K = 64 bf16 each), then BN
-// rows of W (64 K elements: 128 bytes of bf16, or 64 bytes of e4m3 codes, which
-// stay codes in LDS and are widened when a fragment is read).  A 1 KiB DMA
+// One stage of the ring: BM rows of X (128 bytes each, 64 bf16 or 32 fp32 of K),
+// then BN rows of W (as many K elements: 128 bytes of bf16 or fp32, or 64 bytes of
+// e4m3 codes, which stay codes in LDS and are widened when a fragment is read).  A 1 KiB DMA
 // instruction fills 8 rows of 128 bytes or 16 of 64; NP waves share a stage's
 // instructions, each the same number of X and of W ones.
 //
@@ -660,8 +660,10 @@ __global__ __launch_bounds__(256) void splitk_layernorm_kernel(const GemmArgs g,
 // 23 / 29 us; 68 -> 493 TFLOP/s over the four calls, LayerNorms included).
 template <typename WT, int BM, int BN, int NP>
 struct DmaTile {
-  static constexpr bool FP8 = sizeof(WT) == 1;
-  static constexpr int WROW = 64 * (int)sizeof(WT);    // bytes of a W row per stage
+  static constexpr bool FP8 = sizeof(WT) == 1, F32 = sizeof(WT) == 4;
+  static constexpr int BK = F32 ? 32 : 64;             // K elements per stage
+  static constexpr int XS = F32 ? 4 : 2;               // bytes of an X element
+  static constexpr int WROW = BK * (int)sizeof(WT);    // bytes of a W row per stage
   static constexpr int WRPI = 1024 / WROW;             // W rows per instruction
   static constexpr int LA = BM / 8 / NP, LB = BN / WRPI / NP, LPW = LA + LB;  // instructions per wave
   static constexpr int A_BYTES = BM * 128, STAGE_BYTES = A_BYTES + BN * WROW;
@@ -673,8 +675,7 @@ struct DmaTile {
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
       const int rr = (p * LA + j) * 8 + (lane >> 3);
-      a[j] = (const uint8_t*)((const uint16_t*)g.X + (int64_t)min(m0 + rr, g.M - 1) * g.ldx + kbeg +
-                              swz_slot(rr, lane & 7) * 8);
+      a[j] = (const uint8_t*)g.X + ((int64_t)min(m0 + rr, g.M - 1) * g.ldx + kbeg) * XS + swz_slot(rr, lane & 7) * 16;
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
@@ -734,6 +735,34 @@ struct DmaFrags {
   }
 };
 
+// The same for fp32 operands: step j covers k = 8 j .. + 7 of the 32 of a stage,
+// lane half h the four of 16-byte chunk 2 j + h, one v_mfma_f32_32x32x2_f32 per
+// element.
+template <typename T, int FM, int FN>
+struct DmaFragsF32 {
+  f32x4_t a[2][FM], b[2][FN];
+  int a_row, b_row, half, sw;
+  __device__ DmaFragsF32(int m_row, int n_row, int lane)
+      : a_row((m_row + (lane & 31)) * 128), b_row(T::A_BYTES + (n_row + (lane & 31)) * 128), half(lane >> 5),
+        sw(((lane & 31) >> 1) & 7) {}
+  __device__ void load(const uint8_t* stage, int j) {
+    const int kc = ((2 * j + half) ^ sw) << 4;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) a[j & 1][i] = *(const f32x4_t*)(stage + a_row + i * 32 * 128 + kc);
+#pragma unroll
+    for (int i = 0; i < FN; ++i) b[j & 1][i] = *(const f32x4_t*)(stage + b_row + i * 32 * 128 + kc);
+  }
+  __device__ void mfma(int j, f32x16_t (&acc)[FM][FN]) const {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int n = 0; n < FN; ++n)
+          acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j & 1][i][e], b[j & 1][n][e], acc[i][n], 0, 0, 0);
+  }
+};
+
 template <typename WT, int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
   constexpr int NWAVES = WM * WN;
@@ -749,7 +778,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
   const int m0 = tt.x * BM, n0 = tt.y * BN;
   const int kz = blockIdx.z;
   const int kbeg = kz * g.k_per;
-  const int KT = min(g.k_per, g.K - kbeg) / 64;
+  const int KT = min(g.k_per, g.K - kbeg) / T::BK;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -769,7 +798,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  DmaFrags<T, FM, FN> fr(wm * TM, wn * TN, lane);
+  typename std::conditional<T::F32, DmaFragsF32<T, FM, FN>, DmaFrags<T, FM, FN>>::type fr(wm * TM, wn * TN, lane);
   // Waits until k tile t has landed in LDS for every wave: at most
   // (last - t) * LPW of this wave's DMA loads may remain (tiles t+1..last are
   // the younger ones in flight), then a barrier.  The lgkmcnt wait makes
@@ -1888,13 +1917,15 @@ int launch(const GemmArgs& g, hipStream_t s) {
   return check_launch("cbis_gemm");
 }
 
-// fp32 x fp32 tiling.  A 32x32x2 fp32 MFMA occupies its SIMD for 64 cycles,
-// so one wave per SIMD cannot hide its LDS reads and barriers: large grids
-// take 64 x 128 tiles on 8 waves (two per SIMD; config 2 at M = 4096, K =
-// 256: QKV 40.9 -> 24.8 us, MLP up 41.4 -> 25.7 against 128 x 128 on 4
-// waves), and grids with fewer than 4 workgroups of 4 waves per CU split K
-// into up to 4 parts when the caller gives the workspace (config 2, M = 512:
-// MLP down 35.5 -> 14.2 us, the K = 256 shapes 13 -> 9.4-11.7 us).
+// fp32 x fp32 tiling.  A 32x32x2 fp32 MFMA occupies its SIMD for 64 cycles, so
+// several workgroups per CU have to hide each other's LDS reads and barriers:
+// 64 x 64 tiles on 4 waves, with K split into up to 4 parts (when the caller
+// gives the workspace) while that leaves under 4 workgroups per CU (d 256, M =
+// 512, MLP down: 35.5 us whole, 14.2 split), or 64 x 128 tiles on 8 waves where
+// their rounds come out shorter: a CU's share of 64 x 64 tiles against 1.9 times
+// its share of 64 x 128 ones, both rounded up (M = 4096, qkv, 768 or 384 tiles:
+// 18.1 / 22.2 us; MLP up, 1024 or 512: 23.8 / 23.9; d 2048, M = 1216, MLP up, 2560
+// or 1280: 368 / 353).
 struct F32Plan {
   bool wide;  // 64 x 128 on 8 waves; else 64 x 64 (32 x 64 for M <= 32) on 4 waves
   int ksplit = 1;
@@ -1903,17 +1934,17 @@ struct F32Plan {
 
 F32Plan plan_f32(int M, int N, int K) {
   F32Plan p;
-  p.wide = cdiv(M, 128) * cdiv(N, 128) >= 192;
   p.k_per = K;
-  if (p.wide) return p;
   const int64_t tiles = M <= 32 ? cdiv(M, 32) * cdiv(N, 64) : cdiv(M, 64) * cdiv(N, 64);
   const int kt = K / 32;
   // A grid that already gives every CU a workgroup splits only deep K (each
   // part >= 8 K tiles): config 2's out-projection at M = 4096 (256 tiles,
   // K = 256) measured 13.5 us whole and 17.3 in two parts.
   const int min_kt = tiles >= kCUs ? 8 : 4;
-  const int ks = (int)std::min<int64_t>({4, (4 * kCUs) / std::max<int64_t>(1, tiles), kt / min_kt});
-  if (ks <= 1) return p;
+  int ks = (int)std::min<int64_t>({4, (4 * kCUs) / std::max<int64_t>(1, tiles), kt / min_kt});
+  ks = std::max(ks, 1);
+  p.wide = M > 32 && 1.9 * cdiv(cdiv(M, 64) * cdiv(N, 128), kCUs) < (double)cdiv(tiles * ks, kCUs) / ks;
+  if (p.wide || ks == 1) return p;
   const int per = (kt + ks - 1) / ks;
   p.ksplit = (kt + per - 1) / per;
   p.k_per = per * 32;
@@ -2137,6 +2168,13 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
       g.k_per = p.k_per;
       g.partial = (float*)d->workspace;
     }
+    // M > 64.  Direct-to-LDS loads where W's rows are 16-byte aligned (X's always are):
+    // no staging registers, no LDS stores (d 256, register-staged -> direct: M =
+    // 512 qkv / out / up / down 10.9 / 10.1 / 11.9 / 14.4 -> 9.7 / 8.6 / 10.6 / 11.5 us,
+    // M = 4096 22.2 / 17.8 / 24.1 / 37.0 -> 18.1 / 15.1 / 23.9 / 32.8, LayerNorms and
+    // reduces included).  Two slots: three and four measured 2-4% slower.
+    if (((uintptr_t)d->W & 15u) == 0 && d->ldw % 4 == 0)
+      return p.wide ? launch_dma<float, 64, 128, 2, 4, 2>(g, s) : launch_dma<float, 64, 64, 2, 2, 2>(g, s);
     return dispatch<float, float>(g, s);
   }
   // The direct-to-LDS path needs 16-byte aligned rows of both operands.

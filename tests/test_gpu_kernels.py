@@ -129,6 +129,35 @@ def test_gemm_fp32_c2(cbis, oracle, dev, M, shape, ws):
     assert err < FP32_TOL, err
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 8, 32), (65, 130, 64), (129, 64, 96), (300, 200, 1056), (512, 328, 4096),
+                                   (2050, 1028, 96)])
+def test_gemm_fp32_tiles(cbis, oracle, dev, M, N, K):
+    """fp32 tiles above 64 rows with partial tiles in M and N, one stage and
+    many, split K and whole, 64 and 128 columns a tile: W rows on 16 bytes are
+    loaded straight to LDS, rows on 8 bytes through registers; both add in the
+    same order, so they agree to the bit."""
+    import torch
+    x = oracle.normal(71, 1, M * K).reshape(M, K)
+    w = oracle.normal(71, 2, N * K, 0.02).reshape(N, K)
+    b = oracle.normal(71, 3, N, 0.02)
+    X, B = to_dev(x, dev), to_dev(b, dev)
+    pool = torch.empty(N * K + 2, dtype=torch.float32, device=dev)
+    rows = _sample_rows(M, 256, M)
+    ref = oracle.gemm(x[rows], w, bias=b)
+    # fp32 sums of K products in any order: |err| <= (K + 2) 2^-24 sum |x w|
+    tol = (K + 2) * 2.0 ** -24 * (np.abs(x[rows]) @ np.abs(w.T) + np.abs(b))
+    for ws in (False, True):
+        got = []
+        for off in (0, 2):
+            W = pool[off:off + N * K].view(N, K)
+            W.copy_(torch.from_numpy(w))
+            Y = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+            _gemm(cbis, M, N, K, X, cbis.F32, W, cbis.F32, Y, cbis.F32, bias=B, workspace=ws)
+            got.append(Y.cpu().numpy())
+        assert np.array_equal(got[0], got[1])
+        assert (np.abs(got[0][rows] - ref) <= tol).all()
+
+
 @pytest.mark.parametrize("M", [64, 512, 4096])
 @pytest.mark.parametrize("shape", C2_SHAPES, ids=lambda s: s[0])
 def test_gemm_bf16_c2(cbis, oracle, dev, M, shape):
