@@ -267,7 +267,7 @@ __device__ inline int xcd_contiguous(int bid, int nwg) {
 
 __device__ inline int swz(int row, int chunk) { return row * 128 + (swz_slot(row, chunk) << 4); }
 
-template <int BM, int BN, int WM, int WN, int FM, int FN>
+template <int BM, int BN, int WM, int WN, int WK = 1, int FM, int FN>
 __device__ inline void epilogue_parked(const GemmArgs& g, int kz, uint8_t* smem, const f32x16_t (&acc)[FM][FN],
                                        int m0, int n0);
 // LDS bytes epilogue_parked needs for a BM x BN tile.
@@ -704,7 +704,7 @@ struct DmaFrags {
   bf16x8_t a[2][FM];
   uint4 b[2][FN];  // bf16: per k step; fp8: 16 codes, per pair of k steps
   int a_row, b_row, half, sw, sw4;  // sw, sw4: swizzle keys of every row this lane reads (l32 plus multiples of 32)
-  __device__ DmaFrags(int m_row, int n_row, int lane)
+  __device__ DmaFrags(int m_row, int n_row, int lane, int = 0)
       : a_row((m_row + (lane & 31)) * 128), b_row(T::A_BYTES + (n_row + (lane & 31)) * T::WROW), half(lane >> 5),
         sw(((lane & 31) >> 1) & 7), sw4(((lane & 31) >> 2) & 3) {}
   __device__ void load(const uint8_t* stage, int ks) {
@@ -737,16 +737,16 @@ struct DmaFrags {
 
 // The same for fp32 operands: step j covers k = 8 j .. + 7 of the 32 of a stage,
 // lane half h the four of 16-byte chunk 2 j + h, one v_mfma_f32_32x32x2_f32 per
-// element.
+// element.  j counts from j0 on.
 template <typename T, int FM, int FN>
 struct DmaFragsF32 {
   f32x4_t a[2][FM], b[2][FN];
-  int a_row, b_row, half, sw;
-  __device__ DmaFragsF32(int m_row, int n_row, int lane)
-      : a_row((m_row + (lane & 31)) * 128), b_row(T::A_BYTES + (n_row + (lane & 31)) * 128), half(lane >> 5),
-        sw(((lane & 31) >> 1) & 7) {}
+  int a_row, b_row, chunk0, sw;
+  __device__ DmaFragsF32(int m_row, int n_row, int lane, int j0)
+      : a_row((m_row + (lane & 31)) * 128), b_row(T::A_BYTES + (n_row + (lane & 31)) * 128),
+        chunk0(2 * j0 + (lane >> 5)), sw(((lane & 31) >> 1) & 7) {}
   __device__ void load(const uint8_t* stage, int j) {
-    const int kc = ((2 * j + half) ^ sw) << 4;
+    const int kc = ((2 * j + chunk0) ^ sw) << 4;
 #pragma unroll
     for (int i = 0; i < FM; ++i) a[j & 1][i] = *(const f32x4_t*)(stage + a_row + i * 32 * 128 + kc);
 #pragma unroll
@@ -763,9 +763,13 @@ struct DmaFragsF32 {
   }
 };
 
-template <typename WT, int BM, int BN, int WM, int WN, int STAGES>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
-  constexpr int NWAVES = WM * WN;
+// WK = 2: two groups of WM WN waves each sum half of every stage's k steps of the
+// whole tile and meet in the epilogue.
+template <typename WT, int BM, int BN, int WM, int WN, int STAGES, int WK>
+__global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_dma_kernel(const GemmArgs g) {
+  constexpr int NWAVES = WM * WN * WK;
+  constexpr int STEPS = 4 / WK;  // k steps of a stage per wave (double-buffered fragments: an even number)
+  static_assert(WK == 1 || (WK == 2 && sizeof(WT) == 4), "wave groups over K");
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int FM = TM / 32, FN = TN / 32;
   typedef DmaTile<WT, BM, BN, NWAVES> T;
@@ -783,7 +787,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, wn = wave / WM;
+  const int kg = wave / (WM * WN), wm = wave % WM, wn = wave % (WM * WN) / WM;
 
   const T src(g, wave, lane, m0, n0, kbeg);
   const uint32_t lds0 =
@@ -798,7 +802,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  typename std::conditional<T::F32, DmaFragsF32<T, FM, FN>, DmaFrags<T, FM, FN>>::type fr(wm * TM, wn * TN, lane);
+  typename std::conditional<T::F32, DmaFragsF32<T, FM, FN>, DmaFrags<T, FM, FN>>::type fr(wm * TM, wn * TN, lane,
+                                                                                              STEPS * kg);
   // Waits until k tile t has landed in LDS for every wave: at most
   // (last - t) * LPW of this wave's DMA loads may remain (tiles t+1..last are
   // the younger ones in flight), then a barrier.  The lgkmcnt wait makes
@@ -824,8 +829,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
   for (int kt = 0; kt < KT; ++kt) {
     const uint8_t* stage = smem + (kt % STAGES) * STAGE_BYTES;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks < 3) {
+    for (int ks = 0; ks < STEPS; ++ks) {
+      if (ks < STEPS - 1) {
         fr.load(stage, ks + 1);
       } else if (kt + 1 < KT) {
         await_tile(kt + 1, min(KT - 1, kt + STAGES - 1));
@@ -836,14 +841,14 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmAr
     }
   }
 
-  epilogue_parked<BM, BN, WM, WN>(g, kz, smem, acc, m0, n0);
+  epilogue_parked<BM, BN, WM, WN, WK>(g, kz, smem, acc, m0, n0);
 }
 
-template <typename WT, int BM, int BN, int WM, int WN, int STAGES>
+template <typename WT, int BM, int BN, int WM, int WN, int STAGES, int WK = 1>
 int launch_dma(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = cdiv(g.M, BM) * cdiv(g.N, BN);
-  gemm_bf16_dma_kernel<WT, BM, BN, WM, WN, STAGES>
-      <<<dim3((unsigned)tiles, 1, g.ksplit), WM * WN * 64, 0, s>>>(with_vec(g));
+  gemm_bf16_dma_kernel<WT, BM, BN, WM, WN, STAGES, WK>
+      <<<dim3((unsigned)tiles, 1, g.ksplit), WM * WN * WK * 64, 0, s>>>(with_vec(g));
   return check_launch("cbis_gemm(bf16)");
 }
 
@@ -1070,25 +1075,38 @@ __device__ inline void epilogue_rows(const GemmArgs& g, int kz, const float* til
 // parked tile it covers 4-8 rows x 256-512 bytes (16 bytes a lane), a
 // quarter of the instructions for the same bytes.  smem needs
 // BM * (BN + 8) * 4 bytes; the caller's K loop must be done with it.
-template <int BM, int BN, int WM, int WN, int FM, int FN>
+// With WK = 2 the waves WM WN .. 2 WM WN - 1 hold the second summand of the tile:
+// they park first and the others add theirs in place.
+template <int BM, int BN, int WM, int WN, int WK, int FM, int FN>
 __device__ inline void epilogue_parked(const GemmArgs& g, int kz, uint8_t* smem, const f32x16_t (&acc)[FM][FN],
                                        int m0, int n0) {
   constexpr int TM = BM / WM, TN = BN / WN, PITCH = BN + 8;
   static_assert(FM * 32 == TM && FN * 32 == TN, "accumulator blocks");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % WM, wn = wave / WM;
+  const int kg = wave / (WM * WN), wm = wave % WM, wn = wave % (WM * WN) / WM;
   const int half = lane >> 5, l32 = lane & 31;
   float* tile = (float*)smem;
+  auto park = [&](bool add) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          float* t = tile + (wm * TM + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3)) * PITCH + wn * TN + j * 32 + l32;
+          *t = add ? acc[i][j][e] + *t : acc[i][j][e];
+        }
+  };
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        tile[(wm * TM + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3)) * PITCH + wn * TN + j * 32 + l32] = acc[i][j][e];
+  if constexpr (WK == 2) {
+    if (kg == 1) park(false);
+    __syncthreads();
+    if (kg == 0) park(true);
+  } else {
+    park(false);
+  }
   __syncthreads();
-  epilogue_rows<BM, BN, WM * WN * 64>(g, kz, tile, PITCH, m0, n0, tid);
+  epilogue_rows<BM, BN, WM * WN * WK * 64>(g, kz, tile, PITCH, m0, n0, tid);
 }
 
 // Channel scale and bias of the greedy epilogue's columns for lane j of a
@@ -1951,6 +1969,20 @@ F32Plan plan_f32(int M, int N, int K) {
   return p;
 }
 
+// Whether a call that plan_f32 would split, with a reduce launch of its own (not
+// folded into a LayerNorm), instead runs whole on the direct-to-LDS 64 x 64 tiles
+// with two groups of four waves that share each stage's K: as many waves as two
+// parts, without the partials' round trip and the second launch (d 256, M = 65 / 512 /
+// 1000, qkv: 8.6 / 10.0 / 13.7 us split, 7.7 / 7.9 / 8.2 in groups; d 512, M = 200 / 350 /
+// 512 / 1000: 13.4 / 17.3 / 19.8 / 26.6, 12.0 / 12.1 / 12.2 / 22.2).  Three and four parts put more waves on a
+// small grid, so they stay while all of them are in one workgroup per CU (d 512, M =
+// 100, qkv: 9.9 us); so does any split of K past 512, where the matrix time that the
+// parts spread over idle CUs outweighs the reduce's 5 us.
+bool f32_wave_groups(const F32Plan& p, int M, int N, int K) {
+  return p.ksplit > 1 && M > 32 && K <= 512 &&
+         (p.ksplit == 2 || cdiv(M, 64) * cdiv(N, 64) * p.ksplit > kCUs);
+}
+
 // Picks a tile shape from the problem size: the largest tile that still
 // gives the 256 CUs at least about one workgroup each.
 template <typename XT, typename WT>
@@ -2163,6 +2195,9 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
   if (f32) {
     const F32Plan p = plan_f32(d->M, d->N, d->K);
     const size_t need = (size_t)p.ksplit * d->M * d->N * sizeof(float);
+    const bool dma = ((uintptr_t)d->W & 15u) == 0 && d->ldw % 4 == 0;
+    if (dma && !fused_reduce && f32_wave_groups(p, d->M, d->N, d->K))
+      return launch_dma<float, 64, 64, 2, 2, 2, 2>(g, s);
     if (!amax && p.ksplit > 1 && d->workspace && d->workspace_bytes >= need) {
       g.ksplit = p.ksplit;
       g.k_per = p.k_per;
@@ -2173,7 +2208,7 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
     // 512 qkv / out / up / down 10.9 / 10.1 / 11.9 / 14.4 -> 9.7 / 8.6 / 10.6 / 11.5 us,
     // M = 4096 22.2 / 17.8 / 24.1 / 37.0 -> 18.1 / 15.1 / 23.9 / 32.8, LayerNorms and
     // reduces included).  Two slots: three and four measured 2-4% slower.
-    if (((uintptr_t)d->W & 15u) == 0 && d->ldw % 4 == 0)
+    if (dma)
       return p.wide ? launch_dma<float, 64, 128, 2, 4, 2>(g, s) : launch_dma<float, 64, 64, 2, 2, 2>(g, s);
     return dispatch<float, float>(g, s);
   }

@@ -158,6 +158,31 @@ def test_gemm_fp32_tiles(cbis, oracle, dev, M, N, K):
         assert (np.abs(got[0][rows] - ref) <= tol).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 8, 256), (100, 130, 256), (512, 768, 256), (1000, 768, 256), (130, 516, 288),
+                                   (200, 1536, 512), (350, 1540, 480), (700, 1536, 512), (129, 64, 512)])
+def test_gemm_fp32_wave_groups(cbis, oracle, dev, M, N, K):
+    """fp32 calls whose split K is at most two parts, or fills the CUs, up to K =
+    512: one launch of tiles on two wave groups, which needs no workspace (the
+    same bits with and without it); the last shape keeps its four parts."""
+    import torch
+    x = oracle.normal(72, 1, M * K).reshape(M, K)
+    w = oracle.normal(72, 2, N * K, 0.02).reshape(N, K)
+    b = oracle.normal(72, 3, N, 0.02)
+    r = oracle.normal(72, 4, M * N).reshape(M, N)
+    X, W, B, R = (to_dev(t, dev) for t in (x, w, b, r))
+    rows = _sample_rows(M, 256, M)
+    ref = oracle.gemm(x[rows], w, bias=b, residual=r[rows])
+    # fp32 sums of K products, a bias and a residual in any order
+    tol = (K + 3) * 2.0 ** -24 * (np.abs(x[rows]) @ np.abs(w.T) + np.abs(b) + np.abs(r[rows]))
+    got = []
+    for ws in (False, True):
+        Y = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+        _gemm(cbis, M, N, K, X, cbis.F32, W, cbis.F32, Y, cbis.F32, bias=B, residual=R, workspace=ws)
+        got.append(Y.cpu().numpy())
+        assert (np.abs(got[-1][rows] - ref) <= tol).all()
+    assert np.array_equal(got[0], got[1]) or (M, N) == (129, 64)
+
+
 @pytest.mark.parametrize("M", [64, 512, 4096])
 @pytest.mark.parametrize("shape", C2_SHAPES, ids=lambda s: s[0])
 def test_gemm_bf16_c2(cbis, oracle, dev, M, shape):
