@@ -553,17 +553,18 @@ __device__ inline float2 halves(float v) {
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 
-// Workgroups from prefill_blocks on run the decode rows' split merge
-// (decode_merge over merge_rows rows) instead: the merge then shares the
-// prefill launch, which is independent of it, in place of a launch of its own.
+// LDS of a workgroup: per wave a V tile [key][dim], and the waves' states for
+// the merge.
 template <int HPW>
-__global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_kernel(const PrefillArgs a,
-                                                                               const DecodeArgs merge, int merge_rows,
-                                                                               unsigned prefill_blocks) {
-  if (blockIdx.x >= prefill_blocks) {
-    decode_merge(merge, merge_rows, (int64_t)(blockIdx.x - prefill_blocks) * blockDim.x + threadIdx.x);
-    return;
-  }
+struct PrefillLds {
+  __attribute__((aligned(16))) uint8_t vt[HPW * kPrefillWaves][32 * kHD * 2];
+  float pm[HPW][kPrefillWaves][kQG][64], pl[HPW][kPrefillWaves][kQG][64];
+  f32x16_t po[HPW][kPrefillWaves - 1][kQG][64];
+};
+
+// One workgroup's tile and heads, by its first HPW * kPrefillWaves waves.
+template <int HPW>
+__device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillLds<HPW>& lds) {
   const int lane = threadIdx.x & 63;
   const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: block tests and page ids per wave
   const int wave = wave_id % kPrefillWaves;  // key-block lane of this head
@@ -625,8 +626,7 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
   // of key row r in position c ^ ((r >> 2) & 3).  Unswizzled, the 16 lanes
   // of a ds_write_b128 (keys 0..15, one chunk) hit 4 bank groups 4 times
   // each; swizzled, 16 distinct groups.
-  __shared__ __attribute__((aligned(16))) uint8_t vt_all[HPW * kPrefillWaves][32 * kHD * 2];
-  uint8_t* const vt_w = vt_all[wave_id];
+  uint8_t* const vt_w = lds.vt[wave_id];
   auto vpos = [](int key, int chunk) { return key * (kHD * 2) + ((chunk ^ ((key >> 2) & 3)) << 4); };
   // Per query column: o (the P.V accumulator), lacc (every entry the
   // column's sum of the bf16-rounded p: an MFMA of an all-ones A with P^T,
@@ -840,13 +840,11 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
 
   // Merge the waves' (m, l, o) per query column; a wave without blocks has
   // m = -inf and contributes nothing.  Wave 0 always holds key 0.
-  __shared__ float pm_all[HPW][kPrefillWaves][kQG][64], pl_all[HPW][kPrefillWaves][kQG][64];
-  __shared__ f32x16_t po_all[HPW][kPrefillWaves - 1][kQG][64];
 #pragma unroll
   for (int g = 0; g < kQG; ++g) {
-    pm_all[hsub][wave][g][lane] = m[g];
-    pl_all[hsub][wave][g][lane] = lacc[g][0];
-    if (wave > 0) po_all[hsub][wave - 1][g][lane] = o[g];
+    lds.pm[hsub][wave][g][lane] = m[g];
+    lds.pl[hsub][wave][g][lane] = lacc[g][0];
+    if (wave > 0) lds.po[hsub][wave - 1][g][lane] = o[g];
   }
   __syncthreads();
   if (wave != 0) return;
@@ -855,7 +853,7 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
     float l = lacc[g][0];
     float M = m[g];
 #pragma unroll
-    for (int w = 1; w < kPrefillWaves; ++w) M = fmaxf(M, pm_all[hsub][w][g][lane]);
+    for (int w = 1; w < kPrefillWaves; ++w) M = fmaxf(M, lds.pm[hsub][w][g][lane]);
     {
       const float c0 = fast_exp2(m[g] - M);
       l *= c0;
@@ -864,9 +862,9 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
     }
 #pragma unroll
     for (int w = 1; w < kPrefillWaves; ++w) {
-      const float c = fast_exp2(pm_all[hsub][w][g][lane] - M);
-      l += pl_all[hsub][w][g][lane] * c;
-      const f32x16_t ow = po_all[hsub][w - 1][g][lane];
+      const float c = fast_exp2(lds.pm[hsub][w][g][lane] - M);
+      l += lds.pl[hsub][w][g][lane] * c;
+      const f32x16_t ow = lds.po[hsub][w - 1][g][lane];
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[g][i] += ow[i] * c;
     }
@@ -890,6 +888,21 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
   }
 }
 
+// Workgroups from prefill_blocks on run the decode rows' split merge
+// (decode_merge over merge_rows rows) instead: the merge then shares the
+// prefill launch, which is independent of it, in place of a launch of its own.
+template <int HPW>
+__global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_kernel(const PrefillArgs a,
+                                                                               const DecodeArgs merge, int merge_rows,
+                                                                               unsigned prefill_blocks) {
+  if (blockIdx.x >= prefill_blocks) {
+    decode_merge(merge, merge_rows, (int64_t)(blockIdx.x - prefill_blocks) * blockDim.x + threadIdx.x);
+    return;
+  }
+  __shared__ PrefillLds<HPW> lds;
+  prefill_tile<HPW>(a, lds);
+}
+
 // ---------------------------------------------------------------------------
 // Prefill over long contexts: the same tile and MFMA shapes with NWH = 4 waves
 // per head and K/V through LDS.
@@ -906,6 +919,16 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
 // ---------------------------------------------------------------------------
 constexpr int kLongWaves = 4;  // waves per head
 constexpr int kLongRing = 3;   // K/V blocks per key-block lane in LDS: one computed, the others in flight
+// Tiles of up to this many keys run as in paged_prefill_kernel, the workgroup's
+// other waves ending at once: the barriers and LDS reads here cost more than the
+// loads save on them.  One body / the other for whole launches, us a layer (K/V in
+// the last-level cache), 64 heads: 512 rows after 0, 1024, 2048, 3500, 4096, 16384
+// tokens 9.4 / 11.5, 17.6 / 18.4, 25.1 / 25.3, 37.8 / 36.9, 42.0 / 40.1, 139 / 124;
+// 64 rows after 1024, 2048, 3500 13.5 / 15.6, 21.5 / 22.3, 32.8 / 31.7.  7 heads, 64
+// rows after 0, 500, 1024, 2048: 5.2 / 6.2, 9.2 / 9.4, 12.9 / 11.7, 20.7 / 17.1.  A
+// short tile in this kernel takes 0.2 us more than in its own: a larger workgroup
+// is launched.
+constexpr int long_keys(int heads_per_wg) { return heads_per_wg == 2 ? 3072 : 640; }
 // The softmax reference lies this far above the largest score seen when it was
 // set, so that a p within the lazy rescale's headroom is below 2.
 constexpr float kLazyLead = kLazyRescale - 1.f;
@@ -944,6 +967,11 @@ __global__ __launch_bounds__(HPW * kLongWaves * 64, 2) void paged_prefill_long_k
   const int kv_end = min(pos0 + nvalid, a.max_kv);  // keys [0, kv_end) needed by the tile
 
   __shared__ __attribute__((aligned(1024))) uint8_t ring_all[NWH * R * BLOCK];
+  if (kv_end <= long_keys(HPW)) {
+    static_assert(sizeof(PrefillLds<HPW>) <= sizeof(ring_all), "LDS of a short tile");
+    if (wave_id < HPW * kPrefillWaves) prefill_tile<HPW>(a, *(PrefillLds<HPW>*)ring_all);
+    return;
+  }
   uint8_t* const ring = ring_all + wave * (R * BLOCK);
   const uint32_t ring_lds =
       __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring);
@@ -1841,16 +1869,14 @@ int prefill_launch(const cbis_attn_desc* d, int n_tiles, const int* tiles, hipSt
   a.n_heads = d->n_heads;
   a.max_kv = (int)std::min<int64_t>(d->bt_stride * kPS, 1 << 30);
   a.qscale = kLog2e / sqrtf((float)kHD);
-  // Two heads per workgroup.  Sequences that may be long (the table is as wide as
-  // the longest) take the four-wave kernel where the grid gives no CU a second
-  // two-wave workgroup: its barriers and LDS reads cost more than its loads save
-  // on short ones (64 heads, two waves / four, us a layer: 512 rows after 0, 1024,
-  // 4096, 16384 tokens 9.3 / 11.3, 17.2 / 18.2, 40.9 / 39.2, 198 / 128; 64 rows
-  // after 1024, 16384 13.1 / 15.3, 133 / 118) and it does not fit a CU twice (two
-  // 512-row chunks, 512 workgroups: 14.6 / 24.8).
+  // Two heads per workgroup.  Tiles of more than long_keys(hpw) keys take four
+  // waves a head where the grid gives no CU a second two-wave workgroup (the four-wave one
+  // does not fit a CU twice: two 512-row chunks, 512 workgroups, 14.6 / 24.8 us).
+  // The host knows only the table's width, which bounds the keys: each tile picks
+  // its body by its own.
   const int hpw = d->n_heads % 2 == 0 ? 2 : 1;
   const int64_t pgrid = (int64_t)n_tiles * (d->n_heads / hpw);
-  const bool lng = pgrid <= 256 && d->bt_stride * kPS > 4096;
+  const bool lng = pgrid <= 256 && d->bt_stride * kPS > long_keys(hpw);
   const int block = hpw * (lng ? kLongWaves : kPrefillWaves) * 64;
   const DecodeArgs none = {};
   const int64_t mgrid = merge_rows > 0 ? cdiv((int64_t)merge_rows * m->n_heads * kHD, block) : 0;

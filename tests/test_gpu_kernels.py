@@ -1689,6 +1689,64 @@ def test_prefill_attention_long(cbis, oracle, dev, H, qscale, tile_pages):
     assert same.sum() > 200 and row_rel_err(outs[0][same], outs[1][same]) < LOWP_TOL
 
 
+@pytest.mark.parametrize("H,qscale", [(2, 1.0), (3, 16.0), (8, 4.0)])
+@pytest.mark.parametrize("tile_pages", [0, 8])
+def test_prefill_attention_body_by_keys(cbis, oracle, dev, H, qscale, tile_pages):
+    """A prefill tile's kernel body follows from its own keys, not from the
+    block table's width: tiles of up to 3072 keys (640 with an odd head count)
+    give the same bits under a table of that many keys and beside sequences of
+    8000.  Those past it (the
+    four-wave body) against the fp64 oracle: last key block of 1, 16, 17, 31 and
+    32 keys, a lane of waves with a block fewer and with more than 32, one row
+    and a full tile, and queries that raise the softmax reference after the
+    first block.  NaN past every sequence's end must not reach a row."""
+    import torch
+    seqs = [(0, 1), (0, 64), (40, 9), (576, 64), (640, 1), (1000, 70), (3008, 64), (3072, 1), (3057, 16), (3100, 5), (3105, 31),
+            (4100, 60), (4095, 65), (7950, 50)]  # cached, rows
+    D, g = H * 32, rng(60 + H)
+    kv = [a + n for a, n in seqs]
+    npages = [-(-n // 16) for n in kv]
+    P = sum(npages) + 3
+    perm = g.permutation(P).astype(np.int32)
+    wide = np.zeros((len(seqs), max(npages)), np.int32)
+    kp, vp = (bf16_dev(g.standard_normal((P, 16, H, 32)).astype(np.float32), dev) for _ in range(2))
+    tiles, pos, row_seq, at, row = [], [], [], 0, 0
+    for s, (cached, n) in enumerate(seqs):
+        wide[s, : npages[s]] = perm[at: at + npages[s]]
+        at += npages[s]
+        if kv[s] % 16:
+            for t in (kp, vp):
+                t[0][int(wide[s, npages[s] - 1]), kv[s] % 16:] = float("nan")
+        for r in range(0, n, 64):
+            m = min(64, n - r)
+            ids = [int(wide[s, min(16 * k, cached + r + m - 1) // 16]) for k in range(8)]
+            tiles.append([row + r, m, s, cached + r] + (ids if tile_pages else []))
+        pos += range(cached, cached + n)
+        row_seq += [s] * n
+        row += n
+    assert len(tiles) * (H // 2 if H % 2 == 0 else H) <= 256
+    q = (g.standard_normal((row, D)) * qscale).astype(np.float32)
+    # The kernel's Q: scaled by log2(e) / sqrt(32), then rounded to bf16.
+    c = np.float32(1.4426950408889634) / np.sqrt(np.float32(32))
+    qr = bf16_dev(q * c, dev)[1] / c
+    ref = oracle.paged_attention(qr, kp[1], vp[1], wide[row_seq], np.array(pos, np.int32), H, 32, 16)
+    Q, T = to_dev(q, dev), to_dev(np.array(tiles, np.int32), dev)
+    outs = []
+    limit = 3072 if H % 2 == 0 else 640
+    for width in (wide.shape[1], limit // 16):
+        sel = [i for i, t in enumerate(tiles) if kv[t[2]] <= width * 16]
+        BT, TS = to_dev(np.ascontiguousarray(wide[:, :width]), dev), T[sel].contiguous()
+        out = torch.full((row, D), 7.0, dtype=torch.float32, device=dev)
+        d = _attn_desc(cbis, 0, H, Q, kp[0], vp[0], P, BT, width, None, out, cbis.BF16)
+        d.tile_pages = tile_pages
+        cbis.check(cbis.kernels().cbis_paged_prefill_attention(ctypes.byref(d), len(sel), ptr(TS), stream()))
+        sync()
+        outs.append(out.cpu().numpy())
+    assert row_rel_err(outs[0].reshape(row, -1), ref.reshape(row, -1)) < LOWP_TOL
+    short = np.array([kv[s] <= limit for s in row_seq])
+    assert short.sum() == (273 if H % 2 == 0 else 138) and np.array_equal(outs[0][short], outs[1][short])
+
+
 @pytest.mark.parametrize("H", [1, 8, 12])
 @pytest.mark.parametrize("qdt,odt", [("f32", "f32"), ("bf16", "bf16")])
 def test_chunk_attention_f32(cbis, oracle, dev, H, qdt, odt):
