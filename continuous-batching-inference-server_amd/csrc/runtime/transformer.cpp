@@ -37,6 +37,39 @@ constexpr size_t kMaxGraphs = 64;
 // whole step took 162 us for 8 x 512 logits (147 so) and 568 for 512 x 1000 (503).
 constexpr size_t kStagedLogits = (size_t)4 << 20;
 size_t align_ints(size_t n) { return (n + 3) & ~(size_t)3; }
+
+// The rows of an fp32 step: those of runs of at least kMinPrefillRun consecutive
+// positions of a sequence, and the single ones.
+struct RowMix {
+  int rows = 0, singles = 0;
+  int run_kv = 0, single_kv = 0;  // keys of the longest row of each kind
+  int64_t run_keys = 0;           // sum over the runs of rows x keys of the last row
+};
+
+// Whether the runs of an fp32 step go to the chunk kernel's tiles or stay with the
+// single rows.  In tiles a run's keys are read once per 16 rows, but single rows
+// beside them then cost a launch of their own, and a step of up to 64 rows that
+// could take attention and out-projection in one launch (fusable: while its keys
+// are at most 768) a second one.  As decode rows the runs share those launches:
+// they cost what the step's longest row grows by, and, past 768 keys, little as
+// long as 768-token pieces of all rows (per head block) find an idle CU each.
+// Device time of the 4-layer step, all decode rows / in tiles, us:
+//   no single rows, one launch either way: 9 rows at kv 32 112 / 112, at kv 256
+//     149 / 116; 64 rows at kv 174 272 / 278, at kv 364 296 / 280;
+//   8 rows at kv 200 beside 16 fresh ones 178 / 211, beside 16 after 600 tokens
+//     239 / 224; the rows at kv 50: 8 fresh ones 120 / 120, 8 at kv 308 161 / 147;
+//   8 rows at kv 700 beside 32 fresh ones 309 / 361, beside 8 after 2000 261 / 281;
+//   8 rows at kv 200 beside 8 after 2000, 4000 tokens 261 / 213, 249 / 255;
+//   1 row at kv 4000 beside 48 fresh ones, 48 after 600: 374 / 389, 452 / 403.
+// Above 64 rows the runs always go to tiles (100 rows at kv 50 beside 200 fresh
+// ones: 293 / 234 with the linear calls of that size).
+bool chunk_tiles_pay(const RowMix& r, bool fusable, int head_blocks) {
+  if (r.rows > 64) return true;
+  if (r.singles == 0) return !fusable || r.run_kv > 128 + 2 * r.rows;
+  const int pieces = (std::max(r.run_kv, r.single_kv) + 767) / 768;
+  if ((int64_t)r.rows * head_blocks * pieces > 256) return r.run_keys >= 8192;
+  return r.run_kv > 120 + (fusable ? 5 * r.rows : 0) + 1.2 * r.single_kv && r.run_kv + 6.5 * r.single_kv <= 4700;
+}
 }  // namespace
 
 TransformerRunner::TransformerRunner(const ModelWeights& weights, PagedKVCache& cache, int max_total_rows)
@@ -160,25 +193,38 @@ void TransformerRunner::prepare(int b, const int* tok, const int* pos, const int
     rowbt[i] = cur_idx;
   }
   // Rows: runs of consecutive positions of one sequence go to the MFMA
-  // prefill kernel of the K/V dtype, everything else to the split-KV decode
-  // kernel.  Fp32 steps small enough for the fused attention +
-  // out-projection launch keep all their rows in it while their keys are few:
-  // that saves a launch per layer, and re-reading the keys for every row costs
-  // more than that from about 200 keys on (device time of the 4-layer step, all
-  // rows fused / in tiles: 4 x 16 rows at kv 32 247 / 270 us, 64 rows at kv 64 255 /
-  // 270 and at kv 256 279 / 274, 9 rows at kv 32 112 / 112 and at kv 256 149 / 116).
+  // prefill kernel of the K/V dtype (fp32: where that pays), everything else to
+  // the split-KV decode kernel.
   const bool bf16_kv = cfg_.kv_dtype == CBIS_BF16;
-  int top_pos = 0;
-  for (int i = 0; i < M; ++i) top_pos = std::max(top_pos, pos[i]);
-  const bool prefill_ok = bf16_kv || !(fuse_decode_ && attn_proj_ok_ && M <= 64 && top_pos < 128);
   const int tile_rows = bf16_kv ? kTileRows : CBIS_CHUNK_TILE_ROWS, tile_ints = bf16_kv ? kTileInts : 4;
+  auto run_end = [&](int i) {
+    int j = i + 1;
+    while (j < M && seq[j] == seq[i] && pos[j] == pos[j - 1] + 1) ++j;
+    return j;
+  };
+  bool tiles_ok = true;
+  if (!bf16_kv) {
+    RowMix r;
+    r.rows = M;
+    for (int i = 0, j; i < M; i = j) {
+      j = run_end(i);
+      const int n = j - i, kv = pos[j - 1] + 1;
+      if (n >= kMinPrefillRun) {
+        r.run_kv = std::max(r.run_kv, kv);
+        r.run_keys += (int64_t)n * kv;
+      } else {
+        r.singles += n;
+        r.single_kv = std::max(r.single_kv, kv);
+      }
+    }
+    tiles_ok = chunk_tiles_pay(r, fuse_decode_ && attn_proj_ok_, (cfg_.n_heads + 7) / 8);
+  }
   std::vector<int> drows, tiles;
   int max_kv = 1;
   int64_t sum_kv = 0;
-  for (int i = 0; i < M;) {
-    int j = i + 1;
-    while (j < M && seq[j] == seq[i] && pos[j] == pos[j - 1] + 1) ++j;
-    if (prefill_ok && j - i >= kMinPrefillRun) {
+  for (int i = 0, j; i < M; i = j) {
+    j = run_end(i);
+    if (tiles_ok && j - i >= kMinPrefillRun) {
       const std::vector<int>& pg = cache_.pages(seq[i]);
       for (int r = i; r < j; r += tile_rows) {
         const int nv = std::min(tile_rows, j - r);
@@ -197,7 +243,6 @@ void TransformerRunner::prepare(int b, const int* tok, const int* pos, const int
         sum_kv += pos[r] + 1;
       }
     }
-    i = j;
   }
   // Longest rows first: the decode kernel's workgroups are dispatched in row
   // order, so the long rows' splits start early and the short ones fill the

@@ -327,6 +327,54 @@ def test_fused_decode_matches_two_launches(cbis, wdt, kvdt, H):
     assert runner.last_plan()["fused_attention_proj"] == 0
 
 
+@pytest.mark.parametrize("singles,runs,tiles,fused", [
+    ([200] * 8, [(16, 0)], False, True),        # single rows beside a fresh run: one launch a layer
+    ([700], [(40, 0)], False, True),
+    ([50] * 8, [(8, 400)], True, False),        # the run is much longer than the single rows
+    ([120, 31], [(20, 500), (9, 0)], True, False),
+    ([200], [(8, 100), (7, 500)], False, True),  # seven rows are no run
+    ([1000, 40], [(16, 0)], False, False),      # keys past 768: two launches, the run with the single rows
+    ([], [(9, 240)], True, False),              # runs alone
+    ([], [(9, 100)], False, True),
+    ([], [(40, 100), (24, 0)], False, True),
+    ([40] * 50, [(16, 0)], True, False),        # over 64 rows
+])
+def test_f32_step_rows_in_tiles(cbis, oracle, singles, runs, tiles, fused):
+    """Which kernel the runs of rows of an fp32 step take follows what they
+    cost beside the step's single rows; the logits equal the oracle's either
+    way."""
+    spec = oracle.ModelSpec(vocab=512, n_layers=1, max_seq=2048)
+    cfg, w = _ref_model(cbis, vocab=512, n_layers=1, max_seq=2048)
+    shape = [(1, kv - 1) for kv in singles] + runs  # rows, cached
+    pages = sum(-(-(n + c) // 16) for n, c in shape)
+    cache = cbis.PagedKVCache(1, pages, 16, 8, 32, "f32", pages_per_seq=128)
+    runner = cbis.TransformerRunner(w, cache, 512)
+    om = oracle.OracleModel(oracle.synthetic_weights(spec, seed=0), max_pages=pages)
+    ocache = oracle.PagedKVCacheOracle(pages, pages_per_seq=128)
+    step, ostep = ([], [], []), ([], [], [])
+    ids = oracle.uniform_int(0, 91, sum(n + c for n, c in shape), 0, 511)
+    at = 0
+    for n, c in shape:
+        t = [int(x) for x in ids[at:at + n + c]]
+        at += n + c
+        i, o = cache.allocate_sequence(), ocache.allocate_sequence()
+        for p in range(n + c):
+            assert cache.ensure_capacity(i, p) and ocache.ensure_capacity(o, p)
+        for r in range(0, c, 512):  # the rows before the step
+            p = list(range(r, min(c, r + 512)))
+            runner.forward_step(t[r:r + len(p)], p, [i] * len(p))
+            oracle.forward_step_with_cache(om, ocache, t[r:r + len(p)], p, [o] * len(p))
+        for st, sid in ((step, i), (ostep, o)):
+            st[0].extend(t[c:])
+            st[1].extend(range(c, c + n))
+            st[2].extend([sid] * n)
+    got = runner.forward_step(*step)
+    plan = runner.last_plan()
+    assert (plan["prefill_tiles"] > 0, plan["fused_attention_proj"] == 1) == (tiles, fused)
+    assert plan["decode_rows"] == (len(singles) + sum(n for n, _ in runs if n < 8) if tiles else len(step[0]))
+    assert np.abs(got - oracle.forward_step_with_cache(om, ocache, *ostep)).max() < 1e-4
+
+
 @pytest.mark.parametrize("wdt", ["bf16", "fp8", "f32"])
 def test_packed_checkpoint_round_trip(cbis, tmp_path, wdt):
     """save_packed -> load_packed gives back the same config and the same
