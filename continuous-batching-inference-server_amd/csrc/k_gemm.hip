@@ -1813,11 +1813,12 @@ Bf16Path choose_bf16(int M, int N, int K) {
 // its barrier, LDS reads and MFMA chain -- times the K tiles of a workgroup, so
 // the smallest tile that still fits the round wins, and K is split as far as
 // the round allows: the model is K tiles per workgroup times the tile's time,
-// plus the partials' traffic.  Times per K tile fitted on M = 48..512 of the
-// mid-size layer's four shapes (weights cold; qkv / out / fc1 / fc2 in us, LayerNorms
-// included, before and after: M = 64 bf16 17 / 12.6 / 25 / 28 -> 10 / 9.7 / 12 / 16,
-// M = 192 bf16 16 / 20 / 21 / 37 -> 13 / 11 / 16 / 22, fp8 16 / 18 / 17 / 27 ->
-// 13 / 11 / 14 / 18, M = 512 bf16 20 / 19 / 30 / 41 -> 20 / 16 / 25 / 34).
+// plus what the split costs.  The mid-size layer's four calls (weights cold; qkv / out
+// / fc1 / fc2 in us, LayerNorms included) on the tiles below and so: M = 64 bf16 25 /
+// 13.5 / 26 / 28 -> 13 / 10.6 / 14 / 18, M = 192 bf16 21 / 28 / 22 / 38 -> 14 / 13 / 16 /
+// 23, fp8 16 / 18 / 17 / 27 -> 14 / 12 / 15 / 20, M = 512 bf16 23 / 20 / 29 / 42 -> 22 /
+// 17 / 24 / 34.  N = 256, K = 1024 (MLP down, d 256, cold, with its LayerNorm): M = 512
+// 13.2 -> 8.3, M = 2000 14.2 -> 10.8.
 enum class RoundTile { kNone, k64x64, k64x128, k128x64, k96x128, k128x128 };
 struct RoundPlan {
   RoundTile tile = RoundTile::kNone;
@@ -1828,7 +1829,8 @@ constexpr int kRoundMinK = 1024;  // below, the ring fill costs more than the ke
 constexpr int kSplitMinK = 4096;  // a plain call, whose reduce is a launch of its own, splits K from here on
 
 // max_split: the most K parts (1, or 4: the most the reduce kernels take).
-RoundPlan plan_round(int M, int N, int K, int w_dtype, int max_split) {
+// fused_reduce: the LayerNorm kernel that follows reads the parts.
+RoundPlan plan_round(int M, int N, int K, int w_dtype, int max_split, bool fused_reduce) {
   RoundPlan best;
   best.split.k_per = K;
   if (K < kRoundMinK || K % 64) return best;
@@ -1838,19 +1840,26 @@ RoundPlan plan_round(int M, int N, int K, int w_dtype, int max_split) {
     double bf16_us, fp8_us;  // per K tile of 64
   };
   static constexpr Cand kCands[] = {{RoundTile::k64x64, 64, 64, 0.23, 0.22},
-                                    {RoundTile::k128x64, 128, 64, 0.33, 0.30},
-                                    {RoundTile::k64x128, 64, 128, 0.34, 0.28},
-                                    {RoundTile::k96x128, 96, 128, 0.44, 0.37},
-                                    {RoundTile::k128x128, 128, 128, 0.53, 0.47}};
+                                    {RoundTile::k128x64, 128, 64, 0.34, 0.30},
+                                    {RoundTile::k64x128, 64, 128, 0.35, 0.28},
+                                    {RoundTile::k96x128, 96, 128, 0.43, 0.36},
+                                    {RoundTile::k128x128, 128, 128, 0.51, 0.45}};
   const int kt = K / 64;
-  const double part_us = 8e-6 * M * N / 6.0;  // write and read of one part at 6 TB/s
+  // A split's cost: the parts after the first, written at the end of this kernel and
+  // read at the start of the next, and the reduce's launch (or the longer LayerNorm
+  // kernel).  Fitted, with the times per K tile, on 426 calls with K = 1024..8192,
+  // N = 256..16384 and M = 33..2000, each with its split and whole (with a LayerNorm,
+  // bf16, cold, split in two / whole: N = K = 1024, M = 1216 17.2 / 13.7, M = 700 12.5 /
+  // 11.0, M = 128 8.4 / 9.5; N = 4096, K = 1024, M = 300 20.2 / 16.0).
+  const double part_us = 2.3e-6 * M * N, split_us = fused_reduce ? 0.8 : 4.0;
   double t_best = 1e30;
   for (const Cand& c : kCands) {
     const int64_t tiles = cdiv(M, c.bm) * cdiv(N, c.bn);
     for (int ks = 1; ks <= max_split && tiles * ks <= kCUs; ++ks) {
       const int per = (kt + ks - 1) / ks;
       if (ks > 1 && (per < 8 || (kt + per - 1) / per != ks)) continue;
-      const double t = per * (w_dtype == CBIS_BF16 ? c.bf16_us : c.fp8_us) + ks * part_us;
+      const double t = per * (w_dtype == CBIS_BF16 ? c.bf16_us : c.fp8_us) +
+                       (ks > 1 ? split_us + (ks - 1) * part_us : 0);
       if (t < t_best) {
         t_best = t;
         best.tile = c.tile;
@@ -1886,7 +1895,7 @@ DmaPlan plan_dma(int M, int N, int K, int w_dtype, bool fused_reduce, bool may_s
   const bool deep_wide = choose_bf16(M, N, K) == Bf16Path::kWs160Split;
   if (!deep_wide) {
     const RoundPlan r =
-        plan_round(M, N, K, w_dtype, may_split && (fused_reduce || K >= kSplitMinK) ? 4 : 1);
+        plan_round(M, N, K, w_dtype, may_split && (fused_reduce || K >= kSplitMinK) ? 4 : 1, fused_reduce);
     p.round = r.tile;
     p.split = r.split;
     if (r.tile != RoundTile::kNone) return p;

@@ -181,3 +181,25 @@ def test_abi_validation_without_gpu(cbis):
     assert b"aligned" in K.cbis_last_error()
     assert K.cbis_embed(4, 256, 4096, 4096, cbis.BF16, 4096, 4100, 10, 10, 4096, None) == 1
     assert K.cbis_embed(4, 256, 4096, 4096, cbis.BF16, 4096, 4096, 10, 10, 4104, None) == 1
+
+
+@pytest.mark.parametrize("wdt", ["bf16", "fp8"])
+@pytest.mark.parametrize("M,N,K,ln,parts", [
+    (128, 1024, 1024, True, (2, 2)), (192, 2048, 2048, True, (2, 2)), (65, 2048, 2048, True, (4, 4)),
+    (192, 2048, 8192, True, (4, 4)), (512, 2048, 8192, True, (4, 2)), (512, 1024, 4096, False, (2, 4)),
+    # parts cost more than the K tiles they save
+    (1216, 1024, 1024, True, (1, 1)), (700, 1024, 1024, True, (1, 1)), (1500, 512, 1024, True, (1, 1)),
+    (300, 4096, 1024, True, (1, 1)), (192, 8192, 2048, True, (1, 1)), (128, 16384, 4096, False, (1, 1)),
+    (192, 4096, 4096, False, (1, 1)),
+])
+def test_gemm_split_plans(cbis, wdt, M, N, K, ln, parts):
+    """K parts of calls whose grid fits one round of workgroups, from the
+    workspace they ask for: a split has to save more than its partials and
+    its reduce cost."""
+    d = cbis.GemmDesc()
+    d.M, d.N, d.K, d.ldx, d.ldw, d.ldy = M, N, K, K, K, N
+    d.x_dtype, d.w_dtype, d.y_dtype = cbis.BF16, cbis.DTYPES[wdt], cbis.F32
+    lib = cbis.kernels()
+    size = (lib.cbis_gemm_layernorm_workspace_size if ln else lib.cbis_gemm_workspace_size)(ctypes.byref(d))
+    ks = parts[wdt == "fp8"]
+    assert size == (ks * M * N * 4 if ks > 1 else 0)
