@@ -1896,9 +1896,18 @@ DmaPlan plan_dma(int M, int N, int K, int w_dtype, bool fused_reduce, bool may_s
   if (!deep_wide) {
     const RoundPlan r =
         plan_round(M, N, K, w_dtype, may_split && (fused_reduce || K >= kSplitMinK) ? 4 : 1, fused_reduce);
-    p.round = r.tile;
-    p.split = r.split;
-    if (r.tile != RoundTile::kNone) return p;
+    // One row of 96 or 128-row tiles of bf16 W on more than three quarters of the CUs
+    // streams W at HBM's rate; choose_bf16's three ring slots are faster there than four
+    // (weights cold, four / three: N = 32000, K = 2048, M = 96 34.0 / 31.9 us, M = 128
+    // 36.6 / 35.3; N = 28000, M = 96 30.7 / 30.0.  fp8 W, half the bytes: N = 32000, K =
+    // 4096, M = 96 37.7 / 40.0).
+    const bool stream = w_dtype == CBIS_BF16 && M > 64 && M <= 128 && cdiv(N, 128) > 3 * kCUs / 4 &&
+                        cdiv(N, 128) < kCUs;
+    if (r.tile != RoundTile::kNone && !(stream && r.split.ksplit == 1)) {
+      p.round = r.tile;
+      p.split = r.split;
+      return p;
+    }
   }
   p.split.k_per = K;
   if (may_split) p.split = plan_dma_split(M, N, K);

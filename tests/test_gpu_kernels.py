@@ -1634,6 +1634,13 @@ def test_prefill_attention_lazy_rescale(cbis, oracle, dev, mode):
     assert err_head < LOWP_TOL * 2
 
 
+@pytest.mark.parametrize("M,N", [(65, 24577), (96, 32640), (97, 24700), (128, 25000)])
+def test_gemm_one_row_of_tiles(cbis, oracle, dev, M, N):
+    """bf16 W over most of the CUs with one row of 96 or 128-row tiles: three
+    ring slots; ragged last tile."""
+    test_gemm_one_round_tiles(cbis, oracle, dev, "bf16", M, N, 1024, False)
+
+
 @pytest.mark.parametrize("H,qscale", [(2, 1.0), (3, 16.0), (8, 16.0)])
 @pytest.mark.parametrize("tile_pages", [0, 8])
 def test_prefill_attention_long(cbis, oracle, dev, H, qscale, tile_pages):
