@@ -2068,6 +2068,9 @@ bool greedy_skinny(const cbis_gemm_desc* d) {
   return skinny_path(d) && (d->M <= 32 || !dma_eligible(d) || d->K < kRoundMinK ||
                             choose_bf16(d->M, d->N, d->K) == Bf16Path::kSmall);
 }
+// Calls short enough for a LayerNorm prologue are all among them: it runs in the
+// skinny kernel, and the tokens must not depend on whether it ran inside.
+static_assert(kLnPrologueMaxK < kRoundMinK, "greedy calls with a LayerNorm prologue stay on the skinny kernel");
 
 // Column-tile width of the greedy-mode partials for d's GEMM path: the
 // kernels that reduce in their epilogue are the skinny one (16 columns per
@@ -2185,6 +2188,9 @@ int gemm_run(const cbis_gemm_desc* d, hipStream_t s, GemmArgs& g, float4* amax =
   g.k_per = d->K;
   g.partial = nullptr;
   g.amax = amax;
+  // amax was sized for argmax_tile_cols' tiles; the prologue's kernel writes 16-column ones.
+  CBIS_REQUIRE(!amax || !ln || greedy_skinny(d), CBIS_ERR_UNSUPPORTED,
+               "cbis_layernorm_gemm_argmax: LayerNorm prologue off the skinny path");
   g.amax_ld = amax ? (int)cdiv(d->N, argmax_tile_cols(d)) : 0;
   g.ln_x = ln ? ln->x : nullptr;
   g.ln_ldx = ln ? ln->ldx : 0;
@@ -2397,7 +2403,7 @@ int cbis_layernorm_gemm_argmax(const cbis_gemm_desc* d, const float* x, int64_t 
   CBIS_REQUIRE(d->x_dtype == CBIS_F32 || d->x_dtype == CBIS_BF16, CBIS_ERR_UNSUPPORTED, "%s: x dtype", who);
   CBIS_REQUIRE(ldx >= d->K, CBIS_ERR_INVALID, "%s: ldx %lld < K %d", who, (long long)ldx, d->K);
   if (d->M == 0) return CBIS_OK;
-  if (!ln_prologue_ok(d, x, ldx, ln_gamma, ln_beta)) {
+  if (!greedy_skinny(d) || !ln_prologue_ok(d, x, ldx, ln_gamma, ln_beta)) {
     const int rc = cbis_layernorm(d->M, d->K, x, ldx, ln_gamma, ln_beta, eps, d->x_dtype, (void*)d->X, d->ldx, stream);
     if (rc) return rc;
     return cbis_gemm_argmax(d, next_token, margin, workspace, workspace_bytes, stream);

@@ -203,3 +203,18 @@ def test_gemm_split_plans(cbis, wdt, M, N, K, ln, parts):
     size = (lib.cbis_gemm_layernorm_workspace_size if ln else lib.cbis_gemm_workspace_size)(ctypes.byref(d))
     ks = parts[wdt == "fp8"]
     assert size == (ks * M * N * 4 if ks > 1 else 0)
+
+
+@pytest.mark.parametrize("wdt", ["bf16", "fp8"])
+@pytest.mark.parametrize("M", [1, 33, 48, 64])
+def test_greedy_partials_of_layernorm_calls(cbis, wdt, M):
+    """A greedy call that may take its LayerNorm inside (up to 64 rows, K up to
+    512) sizes its partials for the kernel that writes them, one (value, index)
+    pair of pairs per 16 columns, however many tiles N has."""
+    d = cbis.GemmDesc()
+    d.x_dtype, d.w_dtype, d.y_dtype = cbis.BF16, cbis.DTYPES[wdt], cbis.F32
+    d.M = M
+    for N in (1000, 17000, 33000):
+        for K in (64, 256, 512):
+            d.N, d.K, d.ldx, d.ldw, d.ldy = N, K, K, K, N
+            assert cbis.kernels().cbis_gemm_argmax_workspace_size(ctypes.byref(d)) == M * -(-N // 16) * 16
