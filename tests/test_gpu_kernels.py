@@ -384,10 +384,10 @@ def test_gemm_layernorm_matches_gemm_then_layernorm(cbis, oracle, dev, M, N, K, 
                                          (16, 6144, 2048, (1, 1))])
 def test_gemm_layernorm_skinny_split(cbis, oracle, dev, M, N, K, parts, wdt):
     """Decode-sized cbis_gemm_layernorm (config 5's out-projection and fc2:
-    x += h . W^T * scale + b, then LayerNorm(x)): the skinny kernel splits K
-    into `parts` ranges (its 16-column workgroups alone would not occupy the
-    CUs) and the partials are summed, scaled, biased and added to the
-    residual in the LayerNorm's kernel.  x against the fp64 oracle
+    x += h . W^T * scale + b, then LayerNorm(x)): the skinny kernel, or above
+    32 rows the 64 x 64 tiles, split K into `parts` ranges (the workgroups
+    alone would not occupy the CUs) and the partials are summed, scaled, biased
+    and added to the residual in the LayerNorm's kernel.  x against the fp64 oracle
     (1e-5 relative), the normalised rows against the oracle's LayerNorm of
     the GPU's x (one bf16 rounding), and both against the unsplit cbis_gemm
     then cbis_layernorm (summation order only)."""
@@ -571,8 +571,8 @@ def test_gemm_fp8_weights(cbis, oracle, dev, M):
 
 @pytest.mark.parametrize("M,N,K,gelu,res", [
     (65, 250, 64, True, False),       # 64 x 64 tiles, one K tile, ragged rows and columns
-    (700, 1000, 576, False, True),    # 64 x 64 tiles, three ring slots
-    (200, 1000, 4096, True, False),   # 128 x 128 tiles, split K
+    (700, 1000, 576, False, True),    # 64 x 64 tiles, two ring slots
+    (200, 1000, 4096, True, False),   # one round of wave-specialised 64 x 64 tiles, split K
     (1216, 2050, 512, False, True),   # wave-specialised 96 x 128, ragged last column group
     (300, 8200, 512, True, False),    # wave-specialised 128 x 128
     (1300, 8192, 512, False, False),  # the same, over two tiles per CU
@@ -581,9 +581,10 @@ def test_gemm_fp8_weights(cbis, oracle, dev, M):
     (1216, 2048, 6144, False, True),  # wave-specialised 160 x 256, split K
 ])
 def test_gemm_fp8_tiles(cbis, oracle, dev, M, N, K, gelu, res):
-    """fp8 weights at M > 64 on every direct-to-LDS tile (e4m3 codes in the
-    ring, widened at the fragment read), against the product in 64 bits on
-    sampled rows.  Codes and bf16 X are exact, each of the K + 3 fp32
+    """fp8 weights at M > 64 on the direct-to-LDS tiles (e4m3 codes in the
+    ring, widened at the fragment read; the tiles of one round of workgroups
+    and the two below have tests of their own), against the product in 64 bits
+    on sampled rows.  Codes and bf16 X are exact, each of the K + 3 fp32
     operations of an output (sum, scale, bias, residual) is at most 2^-23 of
     the sum of magnitudes off, GELU (slope <= 1.13) adds 1e-6 relative."""
     import torch
@@ -609,6 +610,21 @@ def test_gemm_fp8_tiles(cbis, oracle, dev, M, N, K, gelu, res):
     assert np.all(np.abs(Y.cpu().numpy()[rows] - ref) <= tol)
 
 
+@pytest.mark.parametrize("M,N,K,gelu,res,bm,slots", [
+    (1050, 1000, 576, True, False, 64, 3),   # 17 x 16 tiles of 64 x 64: over one round, K of 8 tiles or more
+    (1100, 960, 960, False, True, 64, 3),
+    (4090, 1020, 256, False, True, 128, 2),  # 32 x 8 tiles of 128 x 128, short K
+    (4097, 1024, 448, True, False, 128, 2),
+])
+def test_gemm_fp8_dma_tiles(cbis, oracle, dev, M, N, K, gelu, res, bm, slots):
+    """fp8 weights on the two tiles of gemm_bf16_dma_kernel that larger grids of
+    short K take (64 x 64 with three ring slots, 128 x 128)."""
+    t128 = -(-M // 128) * -(-N // 128)
+    assert (bm == 128) == (t128 >= 256) and (t128 < 128 or K < 512) and K < 1024
+    assert bm == 128 or (slots == 3) == (K >= 512 and -(-M // 64) * -(-N // 64) >= 256)
+    test_gemm_fp8_tiles(cbis, oracle, dev, M, N, K, gelu, res)
+
+
 @pytest.mark.parametrize("M,N,K,wdt", [(1216, 8000, 512, "fp8"), (300, 6007, 512, "fp8"), (65, 32000, 2048, "fp8"),
                                        (33, 17000, 1024, "fp8"), (64, 17000, 1024, "bf16")])
 def test_gemm_argmax_tiles(cbis, oracle, dev, M, N, K, wdt):
@@ -622,11 +638,11 @@ def test_gemm_argmax_tiles(cbis, oracle, dev, M, N, K, wdt):
     (33, 252, 1024, False),    # 64 x 64, one row tile
     (65, 2048, 2048, True),    # 64 x 64, split under the LayerNorm
     (130, 6148, 1088, False),  # 128 x 64 (bf16) or 64 x 128 (fp8), ragged both ways, 17 K tiles
-    (300, 2052, 4160, True),   # the same, 65 K tiles in uneven parts
+    (300, 2052, 4160, True),   # 64 x 128, 65 K tiles in uneven parts
     (384, 6144, 1024, False),  # 96 x 128
     (384, 2048, 8192, True),   # 96 x 128, split
     (500, 8192, 1024, False),  # 128 x 128, 256 tiles: the last that fits one round
-    (512, 2048, 8192, False),  # 128 x 128, split, reduce of its own
+    (512, 2048, 8192, False),  # 128 x 128 (bf16) or 64 x 128 (fp8), split, reduce of its own
     (514, 8192, 1024, False),  # past it
 ])
 def test_gemm_one_round_tiles(cbis, oracle, dev, wdt, M, N, K, ln):
@@ -1634,6 +1650,22 @@ def test_prefill_attention_lazy_rescale(cbis, oracle, dev, mode):
     assert err_head < LOWP_TOL * 2
 
 
+@pytest.mark.parametrize("M,N,K,wdt", [
+    (66, 2052, 2112, "bf16"), (66, 2052, 2112, "fp8"),    # 64 x 64
+    (66, 4100, 2112, "bf16"), (610, 1028, 2112, "fp8"),   # 128 x 64
+    (134, 3076, 2112, "bf16"), (66, 4100, 2112, "fp8"),   # 64 x 128
+    (474, 2052, 2112, "bf16"), (134, 4100, 4160, "fp8"),  # 96 x 128
+    (202, 4100, 4160, "bf16"), (202, 4100, 4160, "fp8"),  # 128 x 128
+])
+def test_gemm_one_round_splits(cbis, oracle, dev, M, N, K, wdt):
+    """Every one-round tile with K in three uneven parts, ragged rows and columns."""
+    d = cbis.GemmDesc()
+    d.M, d.N, d.K, d.ldx, d.ldw, d.ldy = M, N, K, K, K, N
+    d.x_dtype, d.w_dtype, d.y_dtype = cbis.BF16, cbis.DTYPES[wdt], cbis.F32
+    assert cbis.kernels().cbis_gemm_layernorm_workspace_size(ctypes.byref(d)) == 3 * M * N * 4
+    test_gemm_one_round_tiles(cbis, oracle, dev, wdt, M, N, K, True)
+
+
 @pytest.mark.parametrize("M,N", [(65, 24577), (96, 32640), (97, 24700), (128, 25000)])
 def test_gemm_one_row_of_tiles(cbis, oracle, dev, M, N):
     """bf16 W over most of the CUs with one row of 96 or 128-row tiles: three
@@ -1644,8 +1676,10 @@ def test_gemm_one_row_of_tiles(cbis, oracle, dev, M, N):
 @pytest.mark.parametrize("H,qscale", [(2, 1.0), (3, 16.0), (8, 16.0)])
 @pytest.mark.parametrize("tile_pages", [0, 8])
 def test_prefill_attention_long(cbis, oracle, dev, H, qscale, tile_pages):
-    """Prefill tiles under a block table of more than 4096 keys (the four-wave
-    kernel) against the fp64 oracle and the same tiles under a narrow table:
+    """Prefill tiles under a block table of more than 4096 keys (the launch in
+    which each tile picks its body by its keys: of these only the last
+    sequence's, and with an odd head count the one before, take four waves a
+    head) against the fp64 oracle and the same tiles under a narrow table:
     one key, last key block of 1, 16, 17, 31 and 32 keys, fewer blocks than
     waves, ids reloaded after 32 blocks of a wave, several tiles, even and odd
     head counts, queries that raise the softmax reference after the first
