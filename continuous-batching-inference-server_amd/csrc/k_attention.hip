@@ -553,6 +553,47 @@ __device__ inline float2 halves(float v) {
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 
+// A lane's part of Q^T as the MFMAs' B operand, bf16: dims 8 half .. + 7 of a query
+// row (first MFMA) and 16 + 8 half .. + 7 (second).
+__device__ inline void prefill_q(const PrefillArgs& a, int row, int head, int half, bf16x8_t& b0, bf16x8_t& b1) {
+  float f[16];
+  if (a.q_bf16) {
+    const uint16_t* qp = (const uint16_t*)a.q + (int64_t)row * a.ldq + head * kHD;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f[e] = bf16_to_f32(qp[half * 8 + e]);
+      f[8 + e] = bf16_to_f32(qp[16 + half * 8 + e]);
+    }
+  } else {
+    const float* qp = (const float*)a.q + (int64_t)row * a.ldq + head * kHD;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f[e] = qp[half * 8 + e];
+      f[8 + e] = qp[16 + half * 8 + e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    b0[e] = (short)f32_to_bf16(f[e] * a.qscale);
+    b1[e] = (short)f32_to_bf16(f[8 + e] * a.qscale);
+  }
+}
+
+// Stores a lane's part of a query row: o[i] * inv is dim 8 (i / 4) + 4 half + i % 4,
+// so dims 8 b + 4 half .. + 3 are one 8-byte (bf16) or 16-byte (fp32) store each
+// (ldo % 4 == 0 and a 16-byte aligned out).
+__device__ inline void prefill_store(const PrefillArgs& a, int row, int head, int half, const f32x16_t& o, float inv) {
+  const int64_t ob = (int64_t)row * a.ldo + head * kHD + 4 * half;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const float v0 = o[4 * b] * inv, v1 = o[4 * b + 1] * inv, v2 = o[4 * b + 2] * inv, v3 = o[4 * b + 3] * inv;
+    if (a.out_bf16)
+      *(uint2*)((uint16_t*)a.out + ob + 8 * b) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+    else
+      *(float4*)((float*)a.out + ob + 8 * b) = make_float4(v0, v1, v2, v3);
+  }
+}
+
 // LDS of a workgroup: per wave a V tile [key][dim], and the waves' states for
 // the merge.
 template <int HPW>
@@ -572,9 +613,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillLds<HP
   const int n_hg = a.n_heads / HPW;
   const int tile = blockIdx.x / n_hg;
   const int head = (blockIdx.x % n_hg) * HPW + hsub;
-  // The tile descriptor is the same for the whole workgroup: read it into
-  // scalar registers, so the tests on it (the causal-mask test per block)
-  // compile to scalar branches rather than exec masking.
   // The tile descriptor is the same for the whole workgroup and the page ids
   // of a 32-key block the same for the whole wave: both are read through the
   // constant address space, i.e. with scalar loads (shorter round trips than
@@ -588,37 +626,14 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillLds<HP
   const int col = lane & 31;  // query index within a group (B / C column)
   const int half = lane >> 5;
 
-  // Q^T of group g as the B operand: lane holds q[32 g + col][half*8 + 0..7]
-  // (MFMA 0) and q[32 g + col][16 + half*8 + 0..7] (MFMA 1), bf16.  Rows past
-  // the tile's end repeat its last row (computed, never stored).
+  // Rows past the tile's end repeat its last row (computed, never stored).
   bf16x8_t qb0[kQG], qb1[kQG];
   int qpos[kQG];
 #pragma unroll
   for (int g = 0; g < kQG; ++g) {
     const int qi = min(32 * g + col, nvalid - 1);
-    const int qr = row0 + qi;
     qpos[g] = pos0 + qi;
-    float f[16];
-    if (a.q_bf16) {
-      const uint16_t* qp = (const uint16_t*)a.q + (int64_t)qr * a.ldq + head * kHD;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        f[e] = bf16_to_f32(qp[half * 8 + e]);
-        f[8 + e] = bf16_to_f32(qp[16 + half * 8 + e]);
-      }
-    } else {
-      const float* qp = (const float*)a.q + (int64_t)qr * a.ldq + head * kHD;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        f[e] = qp[half * 8 + e];
-        f[8 + e] = qp[16 + half * 8 + e];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      qb0[g][e] = (short)f32_to_bf16(f[e] * a.qscale);
-      qb1[g][e] = (short)f32_to_bf16(f[8 + e] * a.qscale);
-    }
+    prefill_q(a, row0 + qi, head, half, qb0[g], qb1[g]);
   }
   const int kv_end = min(pos0 + nvalid, a.max_kv);  // keys [0, kv_end) needed by the tile
 
@@ -868,23 +883,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& a, PrefillLds<HP
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[g][i] += ow[i] * c;
     }
-    // o[g][i]: dim 8*(i/4) + 4*half + (i%4) of query 32 g + col.
-    // Dims 8 b + 4 half .. + 3 are o[g][4 b .. 4 b + 3]: one 8-byte (bf16) or
-    // 16-byte (fp32) store each (ldo % 4 == 0 and a 16-byte aligned out).
     const int qi = 32 * g + col;
-    if (qi < nvalid) {
-      const float inv = 1.f / l;
-      const int64_t ob = (int64_t)(row0 + qi) * a.ldo + head * kHD + 4 * half;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const float v0 = o[g][4 * b] * inv, v1 = o[g][4 * b + 1] * inv, v2 = o[g][4 * b + 2] * inv,
-                    v3 = o[g][4 * b + 3] * inv;
-        if (a.out_bf16)
-          *(uint2*)((uint16_t*)a.out + ob + 8 * b) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
-        else
-          *(float4*)((float*)a.out + ob + 8 * b) = make_float4(v0, v1, v2, v3);
-      }
-    }
+    if (qi < nvalid) prefill_store(a, row0 + qi, head, half, o[g], 1.f / l);
   }
 }
 
@@ -1072,37 +1072,14 @@ __global__ __launch_bounds__(HPW * kLongWaves * 64, 2) void paged_prefill_long_k
     }
   }
 
-  // Q^T of group g as the B operand: lane holds q[32 g + col][half*8 + 0..7]
-  // (MFMA 0) and q[32 g + col][16 + half*8 + 0..7] (MFMA 1), bf16.  Rows past
-  // the tile's end repeat its last row (computed, never stored).
+  // Rows past the tile's end repeat its last row (computed, never stored).
   bf16x8_t qb0[kQG], qb1[kQG];
   int qpos[kQG];
 #pragma unroll
   for (int g = 0; g < kQG; ++g) {
     const int qi = min(32 * g + col, nvalid - 1);
-    const int qr = row0 + qi;
     qpos[g] = pos0 + qi;
-    float f[16];
-    if (a.q_bf16) {
-      const uint16_t* qp = (const uint16_t*)a.q + (int64_t)qr * a.ldq + head * kHD;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        f[e] = bf16_to_f32(qp[half * 8 + e]);
-        f[8 + e] = bf16_to_f32(qp[16 + half * 8 + e]);
-      }
-    } else {
-      const float* qp = (const float*)a.q + (int64_t)qr * a.ldq + head * kHD;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        f[e] = qp[half * 8 + e];
-        f[8 + e] = qp[16 + half * 8 + e];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      qb0[g][e] = (short)f32_to_bf16(f[e] * a.qscale);
-      qb1[g][e] = (short)f32_to_bf16(f[8 + e] * a.qscale);
-    }
+    prefill_q(a, row0 + qi, head, half, qb0[g], qb1[g]);
   }
   pin_pages();
 #pragma unroll
@@ -1328,22 +1305,8 @@ __global__ __launch_bounds__(HPW * kLongWaves * 64, 2) void paged_prefill_long_k
 #pragma unroll
       for (int e = 0; e < 16; ++e) o[g][e] += ow[e] * c;
     }
-    // Dims 8 b + 4 half .. + 3 are o[g][4 b .. 4 b + 3]: one 8-byte (bf16) or
-    // 16-byte (fp32) store each (ldo % 4 == 0 and a 16-byte aligned out).
     const int qi = 32 * g + col;
-    if (qi < nvalid) {
-      const float inv = 1.f / l;
-      const int64_t ob = (int64_t)(row0 + qi) * a.ldo + head * kHD + 4 * half;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const float v0 = o[g][4 * b] * inv, v1 = o[g][4 * b + 1] * inv, v2 = o[g][4 * b + 2] * inv,
-                    v3 = o[g][4 * b + 3] * inv;
-        if (a.out_bf16)
-          *(uint2*)((uint16_t*)a.out + ob + 8 * b) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
-        else
-          *(float4*)((float*)a.out + ob + 8 * b) = make_float4(v0, v1, v2, v3);
-      }
-    }
+    if (qi < nvalid) prefill_store(a, row0 + qi, head, half, o[g], 1.f / l);
   }
 }
 
