@@ -620,7 +620,8 @@ __global__ __launch_bounds__(256) void splitk_layernorm_kernel(const GemmArgs g,
 }
 
 // ---------------------------------------------------------------------------
-// bf16 X times bf16 or fp8 W on a multi-stage LDS ring fed by direct-to-LDS loads.
+// bf16 X times bf16 or fp8 W, and fp32 X times fp32 W, on a multi-stage LDS ring
+// fed by direct-to-LDS loads.
 //
 // Each global_load_lds_dwordx4 moves 16 bytes per lane straight from global
 // memory into LDS at M0 + 16 * lane (no VGPRs, no ds_write): one wave
@@ -849,7 +850,7 @@ int launch_dma(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = cdiv(g.M, BM) * cdiv(g.N, BN);
   gemm_bf16_dma_kernel<WT, BM, BN, WM, WN, STAGES, WK>
       <<<dim3((unsigned)tiles, 1, g.ksplit), WM * WN * WK * 64, 0, s>>>(with_vec(g));
-  return check_launch("cbis_gemm(bf16)");
+  return check_launch("cbis_gemm(direct-to-LDS)");
 }
 
 // ---------------------------------------------------------------------------
@@ -1366,12 +1367,12 @@ int launch_ws(const GemmArgs& g, hipStream_t s) {
   if constexpr (GREEDY) {
     if (g.amax) {
       gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, true><<<dim3((unsigned)tiles, 1, 1), 512, 0, s>>>(g);
-      return check_launch("cbis_gemm(bf16 ws)");
+      return check_launch("cbis_gemm(wave-specialised)");
     }
   }
   gemm_bf16_ws_kernel<WT, BM, BN, STAGES, REGS, WM, false>
       <<<dim3((unsigned)tiles, 1, g.ksplit), 512, 0, s>>>(with_vec(g));
-  return check_launch("cbis_gemm(bf16 ws)");
+  return check_launch("cbis_gemm(wave-specialised)");
 }
 
 // ---------------------------------------------------------------------------
@@ -1758,13 +1759,13 @@ struct SplitPlan {
   int k_per = 0;
 };
 
-// Kernel for a bf16 or fp8 W on the direct-to-LDS paths, from the
-// tile counts (measured on config 4's shapes at M = 1216, TFLOP/s):
-//   < kCUs / 2 tiles of 128 x 128, or K < 512: gemm_bf16_dma_kernel (here only
-//     with K < kRoundMinK: plan_round comes first); with under 8 K tiles the
-//     wave-specialised kernel's ring fill and parked epilogue cost more than
-//     they save (config 2, M = 4096, K = 256: 9.5 / 14.1 us against 10.8 /
-//     19.1);
+// Kernel for a bf16 or fp8 W on the direct-to-LDS paths where plan_round has none:
+// K < kRoundMinK, more than one round of workgroups, deep K on large grids, greedy
+// calls.  From the tile counts (measured on the mid-size layer's shapes at M = 1216,
+// TFLOP/s):
+//   < kCUs / 2 tiles of 128 x 128, or K < 512: gemm_bf16_dma_kernel; with under 8
+//     K tiles the wave-specialised kernel's ring fill and parked epilogue cost more
+//     than they save (d 256, M = 4096, K = 256: 9.5 / 14.1 us against 10.8 / 19.1);
 //   < kCUs tiles and K of 96 tiles of 64 or more: 160 x 256 tiles with
 //     split-K into up to 4 parts, about one workgroup per CU.  With weights
 //     cold in HBM, as in the step, this beats whole-K tilings (fc2 at
@@ -1773,8 +1774,8 @@ struct SplitPlan {
 //     warm, 96 x 128 would be faster);
 //   < kCUs tiles otherwise: wave-specialised 96 x 128 (1 x 4 consumers) when
 //     its tiles need no more rounds than 128 x 128 ones, else 128 x 128
-//     (out-projection: 208 tiles of 96 x 128, 535 TFLOP/s against 466 for
-//     160 tiles of 128 x 128);
+//     (N = K = 2048: 208 tiles of 96 x 128, 535 TFLOP/s against 466 for 160
+//     tiles of 128 x 128);
 //   otherwise the wave-specialised tiling with the least estimated time:
 //     the busiest CU's tiles (tiles spread over kCUs CUs) times a tile's
 //     work, 128 x 256 = 1, 160 x 256 = 1.25, 128 x 128 register-staged = 0.5
@@ -2021,7 +2022,6 @@ int dispatch(const GemmArgs& g, hipStream_t s) {
 // g's split.
 template <typename WT>
 int dispatch_dma(const GemmArgs& g, RoundTile round, hipStream_t s) {
-  const bool split = g.ksplit > 1;
   switch (round) {
     case RoundTile::k64x64: return launch_ws<WT, 64, 64, 4, 0, 2, false>(g, s);
     case RoundTile::k64x128: return launch_ws<WT, 64, 128, 4, 0, 1, false>(g, s);
@@ -2036,18 +2036,19 @@ int dispatch_dma(const GemmArgs& g, RoundTile round, hipStream_t s) {
     case Bf16Path::kWs128: return launch_ws<WT, 128, 128, 3>(g, s);
     case Bf16Path::kWs96: return launch_ws<WT, 96, 128, 3, 0, 1>(g, s);
     case Bf16Path::kWs160Split:
-      return split ? launch_ws<WT, 160, 256, 3, 0, 1>(g, s) : launch_ws<WT, 96, 128, 3, 0, 1>(g, s);
+      return g.ksplit > 1 ? launch_ws<WT, 160, 256, 3, 0, 1>(g, s) : launch_ws<WT, 96, 128, 3, 0, 1>(g, s);
     case Bf16Path::kWs128R:
       if constexpr (sizeof(WT) == 2) return launch_ws<WT, 128, 128, 2, 3>(g, s);
       else return launch_ws<WT, 128, 128, 3>(g, s);
     case Bf16Path::kSmall: break;
   }
-  // Grids with fewer 128 x 128 tiles than CUs run 64 x 64 tiles (4 waves
-  // of 32 x 32): four times the workgroups (config 4's out-projection,
-  // 160 tiles: 28.3 -> 23.4 us).  A third ring slot pays when the grid
-  // fills the CUs and K has 8 or more tiles (config 2's MLP down at
-  // M = 4096, K = 1024: 12.2 -> 10.7 us; at M = 512 it costs 1 us).
-  if (!split && cdiv(g.M, kDmaBM) * cdiv(g.N, kDmaBN) < kCUs) {
+  // Grids with fewer 128 x 128 tiles than CUs run 64 x 64 tiles (4 waves of 32 x 32):
+  // four times the workgroups (weights cold, 128 x 128 / so: N = 768, K = 256, M = 512
+  // 6.4 / 5.0 us, M = 2048 6.5 / 5.6).  Past one round of them, K of 8 tiles or more takes a third ring
+  // slot, which covers weights that come from HBM (two / three slots, us: M = 4096, N
+  // = 256, K = 960 cold 9.9 / 8.4, warm 7.3 / 8.0; M = 2100, N = 512, K = 512 cold 7.1
+  // / 6.9, warm 6.2 / 6.7).
+  if (cdiv(g.M, kDmaBM) * cdiv(g.N, kDmaBN) < kCUs) {
     if (g.K >= 512 && cdiv(g.M, 64) * cdiv(g.N, 64) >= kCUs) return launch_dma<WT, 64, 64, 2, 2, 3>(g, s);
     return launch_dma<WT, 64, 64, 2, 2, 2>(g, s);
   }

@@ -139,14 +139,18 @@ typedef struct cbis_gemm_desc {
 } cbis_gemm_desc;
 
 /* Bytes of workspace that let cbis_gemm use its preferred split-K for this
- * descriptor (0 when it does not split). */
+ * descriptor (0 when no call of this shape splits).  An upper bound: an fp32
+ * call of K <= 512 with W rows on 16 bytes may share K inside its workgroups
+ * instead and write none of it. */
 size_t cbis_gemm_workspace_size(const cbis_gemm_desc* d);
 
 int cbis_gemm(const cbis_gemm_desc* d, cbis_stream_t stream);
 
-/* Bytes of workspace that let cbis_gemm_layernorm split K as it prefers: as
- * cbis_gemm_workspace_size, and for decode-sized calls (M <= 64), whose
- * reduce it folds into its LayerNorm kernel, the skinny kernel's split too. */
+/* Bytes of workspace that let cbis_gemm_layernorm split K as it prefers.  Its
+ * LayerNorm kernel sums the parts, so it splits where cbis_gemm does not --
+ * decode-sized calls (M <= 64) on the skinny kernel, bf16 and fp8 tile calls of
+ * any M from K = 1024 on -- or into other parts: size its workspace with this
+ * query and not with cbis_gemm_workspace_size. */
 size_t cbis_gemm_layernorm_workspace_size(const cbis_gemm_desc* d);
 /* cbis_gemm, then a row LayerNorm of its fp32 output Y [M, N] (gamma / beta
  * of N values, eps) into ln_out (fp32 or bf16, row pitch ld_ln): the step's
@@ -154,7 +158,8 @@ size_t cbis_gemm_layernorm_workspace_size(const cbis_gemm_desc* d);
  * next layer's layernorm_forward at :69, or the final one at :92; likewise the
  * out-projection's :81-82 with :84).  When the
  * GEMM splits K the split reduce and the LayerNorm run as one kernel; the
- * results are those of cbis_gemm followed by cbis_layernorm.  Needs Y fp32
+ * results are those of cbis_gemm followed by cbis_layernorm up to the order of
+ * the fp32 sums (bit for bit where both split K alike).  Needs Y fp32
  * without K/V scatter, N a multiple of 4 and <= 8192. */
 int cbis_gemm_layernorm(const cbis_gemm_desc* d, const float* ln_gamma, const float* ln_beta, float eps,
                         int ln_dtype, void* ln_out, int64_t ld_ln, cbis_stream_t stream);
@@ -333,7 +338,8 @@ int cbis_layernorm(int T, int d_model, const float* X, int64_t ldx, const float*
  * :84-85) in one call.  Decode-sized calls with short rows (the skinny path:
  * M <= 64; K <= 512; x, gamma, beta 16-byte aligned, ldx % 4 == 0) form the
  * normalised rows inside the GEMM instead (one launch, X not written); both
- * ways give the same Y bit for bit.  d->X must be a [M, K] buffer of
+ * ways give the same Y bit for bit, except with bf16 W and 33..64 rows, where
+ * cbis_gemm sums in another order.  d->X must be a [M, K] buffer of
  * d->x_dtype (row stride d->ldx). */
 int cbis_layernorm_gemm(const cbis_gemm_desc* d, const float* x, int64_t ldx, const float* ln_gamma,
                         const float* ln_beta, float eps, cbis_stream_t stream);

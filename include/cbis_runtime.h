@@ -117,7 +117,8 @@ int cbis_runner_last_margins(const cbis_runner* r, float* out, int capacity);
 /* Device time in ms of the last step's forward (no reference counterpart: a
  * diagnostic): two events on the runner's stream around the forward's
  * kernels (the first of which also brings the step's metadata from pinned
- * host memory; a greedy step's last one stores its tokens there). */
+ * host memory; a greedy step's last one stores its tokens there, a
+ * forward_step's of up to 4 MiB of logits the logits). */
 float cbis_runner_last_device_ms(const cbis_runner* r);
 /* Host wall time in ms of the last greedy step's phases (no reference
  * counterpart: a diagnostic): out[0] host preparation of the step's
