@@ -911,11 +911,11 @@ __global__ __launch_bounds__(HPW * kPrefillWaves * 64, 2) void paged_prefill_ker
 // two heads of a workgroup are 128 consecutive bytes of a token, and the two
 // waves that work on one key block (one per head) share its ring slot, one
 // loading K and the other V.  The kernel's long contexts are bound by the L2
-// requests (89% of them hit): with a key per lane in the operand layout, or with
+// requests (87% of them hit): with a key per lane in the operand layout, or with
 // a 64-byte head slice per wave, each line is asked for twice or more (one
 // layer, 512 rows after 16384 tokens, 64 heads: 198 us in paged_prefill_kernel,
 // 164 with four waves per head there, 149 with 64-byte DMA rows, of which the
-// loads alone took 144 and the arithmetic alone 109; 128 so).
+// loads alone took 144 and the arithmetic alone 109; 131 so).
 // ---------------------------------------------------------------------------
 constexpr int kLongWaves = 4;  // waves per head
 constexpr int kLongRing = 3;   // K/V blocks per key-block lane in LDS: one computed, the others in flight
